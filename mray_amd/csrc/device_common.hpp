@@ -141,6 +141,15 @@ template <bool POW2> __device__ __forceinline__ float div_c(float a, float b, fl
         return div_rn(a, b, y);
 }
 
+// whether a volume's voxels are addressed by 32-bit byte offsets formed with
+// 24-bit multiplications (PendingSample's OFF32): up to 4 GiB, rows of up to
+// 16 MiB, up to 2^24 of them
+inline bool offsets_fit(int nx, int ny, int nz, size_t voxel_bytes)
+{
+    const uint64_t rows = (uint64_t)ny * nz, row = (uint64_t)nx * voxel_bytes;
+    return rows * row <= (uint64_t)0xFFFFFFFFu + 1u && rows <= (1u << 24) && row < (1u << 24);
+}
+
 // b > 0 is a power of two whose reciprocal host_reciprocal gives (exactly)
 inline bool exact_pow2(float b)
 {
@@ -164,7 +173,7 @@ inline VolumeView<T> make_volume_view(const T *data, int nx, int ny, int nz, con
 }
 
 __device__ __forceinline__ float voxel_value(float v) { return v; }
-__device__ __forceinline__ float voxel_value(uint8_t v) { return (float)(v / 255.f); }
+__device__ __forceinline__ float voxel_value(uint8_t v) { return byte_unit(v); }
 
 // RegularGrid::sample (src/volume.h:97-123): corner-aligned trilinear with
 // clamp-to-edge indices and the reference's weight order.
@@ -197,14 +206,52 @@ template <typename T> __device__ __forceinline__ float sample_volume(const Volum
            ax * (1.f - ay) * az * rlr + (1.f - ax) * ay * az * lrr + ax * ay * az * rrr;
 }
 
+// v clamped to [0, hi] (v_med3; the ternaries of iclamp compile to two)
+__device__ __forceinline__ int clamp0(int v, int hi)
+{
+    int r;
+    asm("v_med3_i32 %0, %1, 0, %2" : "=v"(r) : "v"(v), "v"(hi));
+    return r;
+}
+
+// Positions on the grid of three coordinates, (p - dmin) / (dmax - dmin) * n
+// per axis as the reference rounds it. POW2: every extent is a power of two,
+// so the division is exact and folds with the multiplication by n (an exact
+// product of the two) into one rounding. Otherwise div_rn with one range check
+// for the three axes (a zero dividend is exact, too).
+template <bool POW2, typename V>
+__device__ __forceinline__ void grid_position(const V &v, float px, float py, float pz, float &ix, float &iy, float &iz)
+{
+    const float ax = px - v.dmin.x, ay = py - v.dmin.y, az = pz - v.dmin.z;
+    if constexpr (POW2)
+    {
+        ix = ax * (v.rext.x * (float)v.nx);
+        iy = ay * (v.rext.y * (float)v.ny);
+        iz = az * (v.rext.z * (float)v.nz);
+        return;
+    }
+    const float ex = v.dmax.x - v.dmin.x, ey = v.dmax.y - v.dmin.y, ez = v.dmax.z - v.dmin.z;
+    float qx = div_rn_core(ax, ex, v.rext.x), qy = div_rn_core(ay, ey, v.rext.y), qz = div_rn_core(az, ez, v.rext.z);
+    const float qm = fmaxf(fmaxf(fabsf(qx), fabsf(qy)), fabsf(qz));
+    const bool nan = !(qx == qx && qy == qy && qz == qz);
+    if (__builtin_expect(min(min(div_rn_key(ax), div_rn_key(ay)), div_rn_key(az)) < kDivRnKeyMin || !(qm <= 0x1p60f) || nan, 0))
+    {
+        qx = ax / ex;
+        qy = ay / ey;
+        qz = az / ez;
+    }
+    ix = qx * (float)v.nx;
+    iy = qy * (float)v.ny;
+    iz = qz * (float)v.nz;
+}
+
 // sample_volume split in two: issue() computes the weights and starts the
 // eight loads, value() combines them later, so that the loads of the next
 // sample are in flight while the current one is used (same arithmetic and
-// result as sample_volume). OFF32: the volume spans at most 4 GiB, so the
-// corners are addressed by 32-bit byte offsets from the base (one scalar
-// base, no 64-bit address arithmetic per load). POW2: every extent of the
-// domain is a power of two, so dividing by it is multiplying by its exact
-// reciprocal.
+// result as sample_volume). OFF32 (offsets_fit): the corners are addressed by
+// 32-bit byte offsets from the base (one scalar base, no 64-bit address
+// arithmetic per load), formed by 24-bit multiply-adds (full rate; a 32-bit
+// multiply issues at a quarter of it). POW2: see grid_position.
 template <typename T, bool OFF32 = false, bool POW2 = false> struct PendingSample
 {
     float ax, ay, az;
@@ -212,42 +259,42 @@ template <typename T, bool OFF32 = false, bool POW2 = false> struct PendingSampl
 
     __device__ __forceinline__ void issue(const VolumeView<T> &v, float px, float py, float pz)
     {
-        const float ipx = div_c<POW2>(px - v.dmin.x, v.dmax.x - v.dmin.x, v.rext.x) * (float)v.nx;
-        const float ipy = div_c<POW2>(py - v.dmin.y, v.dmax.y - v.dmin.y, v.rext.y) * (float)v.ny;
-        const float ipz = div_c<POW2>(pz - v.dmin.z, v.dmax.z - v.dmin.z, v.rext.z) * (float)v.nz;
-        float flx = floorf(ipx), fly = floorf(ipy), flz = floorf(ipz);
+        float ipx, ipy, ipz;
+        grid_position<POW2>(v, px, py, pz, ipx, ipy, ipz);
+        const float flx = floorf(ipx), fly = floorf(ipy), flz = floorf(ipz);
         ax = ipx - flx;
         ay = ipy - fly;
         az = ipz - flz;
-        int xl = (int)flx, yl = (int)fly, zl = (int)flz;
-        int x0 = iclamp(xl, 0, v.nx - 1), x1 = iclamp(xl + 1, 0, v.nx - 1);
-        int y0 = iclamp(yl, 0, v.ny - 1), y1 = iclamp(yl + 1, 0, v.ny - 1);
-        int z0 = iclamp(zl, 0, v.nz - 1), z1 = iclamp(zl + 1, 0, v.nz - 1);
+        const int xl = (int)flx, yl = (int)fly, zl = (int)flz;
+        const int x0 = clamp0(xl, v.nx - 1), y0 = clamp0(yl, v.ny - 1), z0 = clamp0(zl, v.nz - 1);
+        // the clamped upper neighbour is one further where 0 <= xl < nx - 1, else the same voxel
+        const bool fx = (uint32_t)xl < (uint32_t)(v.nx - 1), fy = (uint32_t)yl < (uint32_t)(v.ny - 1),
+                   fz = (uint32_t)zl < (uint32_t)(v.nz - 1);
         const uint32_t sxy = (uint32_t)(v.ny * v.nx);
         if constexpr (OFF32)
         {
             constexpr uint32_t B = sizeof(T);
             const char *base = reinterpret_cast<const char *>(v.data);
-            const uint32_t o0 = ((uint32_t)z0 * sxy + (uint32_t)(y0 * v.nx + x0)) * B;
-            const uint32_t dxb = (uint32_t)(x1 - x0) * B;
-            const uint32_t dyb = (uint32_t)((y1 - y0) * v.nx) * B;
-            const uint32_t o1 = o0 + ((z1 > z0) ? sxy * B : 0u);
+            const uint32_t row = __umul24((uint32_t)z0, (uint32_t)v.ny) + (uint32_t)y0;
+            const uint32_t o0 = __umul24(row, (uint32_t)v.nx * B) + (uint32_t)x0 * B;
+            const uint32_t dxb = fx ? B : 0u, dyb = fy ? (uint32_t)v.nx * B : 0u;
+            const uint32_t o1 = o0 + (fz ? sxy * B : 0u);
+            const uint32_t o2 = o0 + dyb, o3 = o1 + dyb;
             lll = *reinterpret_cast<const T *>(base + o0);
             rll = *reinterpret_cast<const T *>(base + (o0 + dxb));
-            lrl = *reinterpret_cast<const T *>(base + (o0 + dyb));
-            rrl = *reinterpret_cast<const T *>(base + (o0 + dyb + dxb));
+            lrl = *reinterpret_cast<const T *>(base + o2);
+            rrl = *reinterpret_cast<const T *>(base + (o2 + dxb));
             llr = *reinterpret_cast<const T *>(base + o1);
             rlr = *reinterpret_cast<const T *>(base + (o1 + dxb));
-            lrr = *reinterpret_cast<const T *>(base + (o1 + dyb));
-            rrr = *reinterpret_cast<const T *>(base + (o1 + dyb + dxb));
+            lrr = *reinterpret_cast<const T *>(base + o3);
+            rrr = *reinterpret_cast<const T *>(base + (o3 + dxb));
             return;
         }
-        // one 64-bit corner address, the others by 32-bit offsets (the
-        // clamped neighbour is 0 or 1 cell away on each axis)
+        // one 64-bit corner address, the others by 32-bit offsets
         const T *p0 = v.data + ((size_t)z0 * sxy + (uint32_t)(y0 * v.nx + x0));
-        const uint32_t dx = (uint32_t)(x1 - x0);
-        const uint32_t dy = (uint32_t)((y1 - y0) * v.nx);
-        const T *p1 = p0 + ((z1 > z0) ? sxy : 0u);
+        const uint32_t dx = fx ? 1u : 0u;
+        const uint32_t dy = fy ? (uint32_t)v.nx : 0u;
+        const T *p1 = p0 + (fz ? sxy : 0u);
         lll = p0[0];
         rll = p0[dx];
         lrl = p0[dy];

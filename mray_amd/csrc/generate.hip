@@ -19,17 +19,15 @@
 //         (eps); both enter to first order, exactly enough to reproduce the
 //         reference's arithmetic-free result to ~1e-13:
 //             + sum_k [ -delta_k f_k cos(j p_k) + h_k sin(j p_k) / j ].
-//         A node costs cos and sin of its (float) phase and two Chebyshev
-//         recurrences over j (cos and sin of j phi): five operations per
-//         moment (accumulate_node) instead of 2(m-1) sin/cos. gfx950 issues
-//         FP64 FMAs at the rate of unpacked FP32 ones, so the cosine
-//         recurrence and sums (the moments' bulk) and trig_0 (the exact
-//         integral of the reference's lines) are FP64; the sine terms carry
-//         only the first-order ulp corrections and stay FP32. The moments are
-//         rounded to float once. The node's phasor is the previous one turned
-//         by the exact FP64 difference of the two float phases (the
-//         reference's phases jitter by ulps around the uniform grid, so a
-//         fixed step would drift off cos(p_k)). Moments live in registers
+//         Two marches sum these terms. Where the samples resolve the largest
+//         order (almost every ray), the ulp-sized terms become weights of
+//         plain cosines on the ray's uniform phase grid (WeightRing), and a
+//         moment costs one FP64 operation per node (accumulate_blocks); the
+//         other rays are summed node by node from each node's own phasor,
+//         five operations per moment (accumulate_node). gfx950 issues FP64
+//         FMAs at the rate of unpacked FP32 ones, so the cosine sums and
+//         trig_0 (the exact integral of the reference's lines) are FP64; the
+//         moments are rounded to float once. Moments live in registers
 //         (template M >= m); more than 60 are split into chunks over
 //         workgroups (CHUNK).
 #include "device_common.hpp"
@@ -49,6 +47,15 @@ struct GenArgs
     int transform_to_bounds;
     int compact_image;
     float bound_eps;
+    int rays; // which rays a launch of generate_mixed_kernel takes (GenRays)
+};
+
+// the rays of a MIXED launch, by wavefront: every one, or those summed node by
+// node where another launch takes the gridded ones
+enum GenRays : int
+{
+    kRaysAll = 0,
+    kRaysUngridded = 1,
 };
 
 // Sample at t along r (origin + t * dir in float, as the reference).
@@ -188,7 +195,89 @@ __global__ __launch_bounds__(256) void generate_plain_kernel(VolumeView<T> vol, 
 // MIXED
 // ---------------------------------------------------------------------------
 
-// One node's terms for moments j = 1..M-1:
+// The moment sums of a march keep, for every node n of the ray's uniform
+// phase grid q_n, one weight w_n (the stencil below): sc_j = sum_n w_n
+// cos(j q_n), trig_j = sc_j / j^2 up to the ray's first sample. In FP64:
+// gfx950 issues FP64 FMAs at the rate of unpacked FP32 ones.
+//
+// accumulate_blocks takes the cosines as products, j = q P + r:
+//     a_qr += (w T_qP(x)) T_r(x),   x = cos(q_n),
+// with T_r, r < P, and w T_qP by their Chebyshev recurrences, so that a
+// moment costs one operation and a node P + M / P more, instead of two per
+// moment. 2 T_qP T_r = T_qP+r + T_qP-r, so the sums of cosines follow from the
+// sums of products once per ray (untangle_blocks). P near sqrt(M) makes the
+// overhead smallest; slot 0 (moment 0, integrated separately) is not summed.
+template <int M> constexpr int block_width() { return M <= 12 ? 4 : M <= 30 ? 5 : M <= 56 ? 7 : M <= 72 ? 8 : 10; }
+
+template <int M> __device__ __forceinline__ void accumulate_blocks(double (&sc)[M], double w, double x)
+{
+    constexpr int P = block_width<M>();
+    const double x2 = x + x;
+    double T[P + 1];
+    T[0] = 1.0;
+    T[1] = x;
+#pragma unroll
+    for (int r = 2; r <= P; ++r)
+        T[r] = fma(x2, T[r - 1], -T[r - 2]);
+    const double y2 = T[P] + T[P];
+    double z1 = w, z = w;
+#pragma unroll
+    for (int q = 0; q * P < M; ++q)
+    {
+        if (q == 1)
+            z = w * T[P];
+        else if (q > 1)
+        {
+            const double zn = fma(y2, z, -z1);
+            z1 = z;
+            z = zn;
+        }
+#pragma unroll
+        for (int r = 0; r < P; ++r)
+        {
+            const int j = q * P + r;
+            if (j >= M || j == 0)
+                continue;
+            if (r == 0)
+                sc[j] += z;
+            else
+                sc[j] = fma(z, T[r], sc[j]);
+        }
+    }
+}
+
+// sums of cosines from accumulate_blocks' sums of products:
+// sc_qP+r = 2 a_qr - sc_qP-r for q, r >= 1 (the other slots are products with T_0)
+template <int M> __device__ __forceinline__ void untangle_blocks(double (&sc)[M])
+{
+    constexpr int P = block_width<M>();
+#pragma unroll
+    for (int j = P + 1; j < M; ++j)
+        if (j % P != 0)
+            sc[j] = fma(2.0, sc[j], -sc[j / P * P - j % P]);
+}
+
+// The chunk j0 .. j0 + M - 1 of a march whose moments are split into chunks:
+// sc_i += w cos((j0 + i) q_n) by the recurrence from w cos(j0 q_n) and
+// w cos((j0 + 1) q_n) (c0, c1), two operations per moment.
+template <int M> __device__ __forceinline__ void accumulate_chunk(double (&sc)[M], double w, double x, double c0, double c1)
+{
+    const double x2 = x + x;
+    double v1 = w * c0, v = w * c1;
+    sc[0] += v1;
+    sc[1] += v;
+#pragma unroll
+    for (int i = 2; i < M; ++i)
+    {
+        const double n = fma(x2, v, -v1);
+        v1 = v;
+        v = n;
+        sc[i] += v;
+    }
+}
+
+// One node of an exactly summed ray (see the kernel), its terms at its own phase,
+// moments j = 1..M-1:
 //     sc[j] += (d + j^2 e) cos(j phi)   (FP64)
 //     ss[j] += h sin(j phi)             (FP32)
 // the moment being (sc[j] + j ss[j]) / j^2. cos(j phi) by the Chebyshev
@@ -312,17 +401,107 @@ __device__ __forceinline__ void accumulate_node_chunk_c(double (&sc)[M], float (
     }
 }
 
-// CHUNK: the moments are split into chunks of M (more than one thread's
-// registers hold); each chunk's workgroups march the same rays and
-// accumulate moments j0 .. j0 + M - 1. The first chunk is the unchunked
-// kernel (M moments of an image of m > M: it writes moments 0 .. M - 1, the
-// bounds, the ray range and the sample counts, and needs no per-node phasor
-// of j0 phi); the CHUNK kernel runs the later chunks, j0 = (blockIdx.y + 1) M,
-// or j0 = J0C when that is nonzero (the second of two chunks: its weights
-// take literal odd factors, and cos and sin of j0 phi follow the node's
-// phasor by a rotation instead of a sincos per node).
-template <typename T, int M, bool OFF32, bool POW2, bool CHUNK = false, int J0C = 0>
-__global__ __launch_bounds__(256) void generate_mixed_kernel(VolumeView<T> vol, DevCamera cam, GenArgs a,
+// Pending weights of the eight grid nodes around the newest one (the 9-point
+// stencils of the first two derivatives, error (j Delta)^8 / 630 and / 3150 of
+// the term). push adds node k's functional d c + cp c' + cpp c'' and returns
+// the finished weight of node k - 4; A = cpp / Delta^2, B = cp / Delta. The
+// ring moves on by writing each sum into the next slot (no copies).
+struct WeightRing
+{
+    double w[8];
+
+    // r = a b + c with r a register of its own (left to the compiler, each
+    // sum is formed in its old slot's registers and copied over)
+    static __device__ __forceinline__ void fma_to(double &r, double a, double b, double c)
+    {
+        asm("v_fma_f64 %0, %1, %2, %3" : "=v"(r) : "s"(a), "v"(b), "v"(c));
+    }
+
+    __device__ __forceinline__ WeightRing()
+    {
+#pragma unroll
+        for (int i = 0; i < 8; ++i)
+            w[i] = 0.0;
+    }
+
+    __device__ __forceinline__ double push(double d, double A, double B)
+    {
+        constexpr double a0 = -205.0 / 72.0, a1 = 8.0 / 5.0, a2 = -1.0 / 5.0, a3 = 8.0 / 315.0, a4 = -1.0 / 560.0;
+        constexpr double b1 = 4.0 / 5.0, b2 = -1.0 / 5.0, b3 = 4.0 / 105.0, b4 = -1.0 / 280.0;
+        const double out = fma(a4, A, fma(-b4, B, w[0]));
+        fma_to(w[0], a3, A, fma(-b3, B, w[1]));
+        fma_to(w[1], a2, A, fma(-b2, B, w[2]));
+        fma_to(w[2], a1, A, fma(-b1, B, w[3]));
+        fma_to(w[3], a0, A, w[4] + d);
+        fma_to(w[4], a1, A, fma(b1, B, w[5]));
+        fma_to(w[5], a2, A, fma(b2, B, w[6]));
+        fma_to(w[6], a3, A, fma(b3, B, w[7]));
+        w[7] = fma(a4, A, b4 * B);
+        return out;
+    }
+
+    __device__ __forceinline__ double pop()
+    {
+        const double out = w[0];
+#pragma unroll
+        for (int i = 0; i < 7; ++i)
+            w[i] = w[i + 1];
+        w[7] = 0.0;
+        return out;
+    }
+};
+
+// The integral per node. A segment [u, p] of the reference with slope g
+// contributes, with c(phi) = cos(j phi) and rho the line's values at its ends,
+//     (1/j^2) [ g c(p) - rho_p c'(p) - g c(u) + rho_u c'(u) ].
+// Node k gathers the end of segment k (at p_k) and the start of segment k + 1
+// (at u_k+1 = p_k + delta, the reference's p_k+1 - dphi in float). Expanded
+// around the uniform grid q_k = (t_k - t_near) pi / range - pi (p_k = q_k +
+// eps; eps, delta are a few float ulps of the phase, their squares ~1e-13):
+//     d c + cp c' + cpp c''   at q_k,
+//     d   = g_k - g_k+1
+//     cp  = d eps - g_k+1 delta - g_k (width_k - dphi)
+//     cpp = f_k delta
+// On the uniform grid the derivatives are 9-point differences of c at the
+// neighbouring nodes, so a node's terms become weights of plain cosines
+// (WeightRing) and a moment costs one FP64 operation per node (five before:
+// cosine, sine and weight recurrences and two sums). The stencils reach past
+// the ray's ends: c is defined there too. This needs the largest order
+// resolved by the grid, (m - 1) dphi <= 1 (at 1: 1.6e-3 of cp's terms, i.e.
+// ~1e-10 of the moments), and t's float increments uniform (t_far <= 8192 s:
+// where t passes a power of two they change by at most 2^-11): grid_resolves.
+// The wavefronts with a ray that fails it (a few samples for many moments)
+// are summed node by node (!GRID): the terms at p_k itself, cosine sums in
+// FP64 and the ulp-sized sine terms in FP32, five operations per moment. The
+// two are kernels of their own, launched over the same tiles (registers: the
+// sine sums would cost the gridded march a wavefront per SIMD at 30 moments).
+//
+// A pass that records the rays' normalisation is the forward of a gradient
+// (generate_backward) and is summed node by node for every ray: the bounded
+// MESE amplifies the last bit of a moment to up to 1e-2 of the gradient's
+// norm (mixing layers of 60 to 120 voxels: 1 to 9e-3 between two sums that
+// are both within a moment's rounding), so that pass keeps one rounding.
+//
+// CHUNK: more moments than one thread's registers hold are split into chunks
+// of M; each chunk's workgroups march the same rays and accumulate moments
+// j0 .. j0 + M - 1. The first chunk is the unchunked kernel (M moments of an
+// image of m > M: it writes moments 0 .. M - 1, the bounds, the ray range and
+// the sample counts); the CHUNK kernel runs the later ones,
+// j0 = (blockIdx.y + 1) M.
+// J0C: a chunk start known at compile time (!GRID).
+//
+// Measured (1024^3 f32, 1024 x 1024 rays, 50 moments): 11.6 ms node by node,
+// 8.1 ms gridded, 207 instead of 341 VALU instructions per node, 84 % of the
+// issue slots; 2048 x 2048 x 1920 u8, 2048 x 2048 rays, 100 moments: 132 and
+// 77 ms (the bytes' divisions and the corner addresses are a third of that
+// gain). Bound by VALU issue, then by load latency at two wavefronts per SIMD.
+__device__ __forceinline__ bool grid_resolves(int m, float dphi, float t_near, float t_far, float s)
+{
+    return (float)(m - 1) * dphi <= 1.0f && t_far <= 8192.0f * s && t_near + s < t_far;
+}
+
+template <typename T, int M, bool OFF32, bool POW2, bool CHUNK, bool GRID, int J0C>
+__global__ __launch_bounds__(256, 2) void generate_mixed_kernel(VolumeView<T> vol, DevCamera cam, GenArgs a,
                                                              float *__restrict__ out, uint32_t *__restrict__ bounds,
                                                              int32_t *__restrict__ samples,
                                                              float2 *__restrict__ ray_range)
@@ -340,7 +519,7 @@ __global__ __launch_bounds__(256) void generate_mixed_kernel(VolumeView<T> vol, 
     const int m = a.m;
     const int j0 = CHUNK ? (J0C ? J0C : (int)(blockIdx.y + 1) * M) : 0;
     const bool first_chunk = !CHUNK;
-    const int jend = CHUNK ? min(m, j0 + M) : m;
+    const int jend = CHUNK ? min(m, j0 + M) : min(m, M);
     Ray r = pixel_ray(cam, a.W, a.H, x, y);
     float t_near, t_far;
     bool hit = intersect_aabb(r, vol.dmin, vol.dmax, t_near, t_far);
@@ -349,6 +528,8 @@ __global__ __launch_bounds__(256) void generate_mixed_kernel(VolumeView<T> vol, 
     float *mo = out + pix * (size_t)m;
     if (!(hit && (t_far > 0)))
     {
+        if (!GRID && a.rays == kRaysUngridded)
+            return; // written by the gridded launch
         if (!(a.transform_to_bounds && a.compact_image))
             for (int j = j0; j < jend; ++j)
                 mo[j] = 0.f;
@@ -367,67 +548,36 @@ __global__ __launch_bounds__(256) void generate_mixed_kernel(VolumeView<T> vol, 
     const float s = a.step;
     const float pi_trange_inv = (float)(kPi / (double)(t_far - t_near));
     const float dphi = (float)(kPi * (double)(s / (t_far - t_near)));
+    // by wavefront: whether its rays are gridded
+    const bool gridded = !__any(!grid_resolves(m, dphi, t_near, t_far, s));
+    if (GRID ? !gridded : (gridded && a.rays == kRaysUngridded))
+        return;
 
     float t = t_near;
-    float f_prev = sample_at(vol, r, t, a);
-    const float f_first = f_prev;
-    float lo = rmin(1.f, f_prev), hi = rmax(0.f, f_prev);
+    const float f_first = sample_at(vol, r, t, a);
+    float lo = rmin(1.f, f_first), hi = rmax(0.f, f_first);
     int ns = 1;
 
     // phase of node 0: start of the first segment, p_1 - dphi (or -pi when the
     // ray has no interior sample), as update_moments forms p_prev.
-    float node_phase;
+    float phase0;
     if (t + s < t_far)
     {
         float t1 = t + s;
         float p1 = (float)((double)((t1 - t_near) * pi_trange_inv) - kPi);
-        node_phase = p1 - dphi;
+        phase0 = p1 - dphi;
     }
     else
-        node_phase = (float)(-kPi);
-    // cos and sin of the node phase (FP64, of the float phase)
-    double zs, zc;
-    sincos_small((double)node_phase, zs, zc);
-    const double z0s = zs, z0c = zc;
-    // CHUNK: cos and sin of j0 phi and (j0 + 1) phi at the current node (the
-    // product j0 phi is exact in FP64)
-    const double j0d = (double)j0;
-    double kc = 1.0, ks = 0.0, kc1 = zc, ks1 = zs;
-    auto chunk_start = [&](float ph) {
-        if constexpr (CHUNK)
-        {
-            sincos_small(j0d * (double)ph, ks, kc);
-            kc1 = fma(kc, zc, -ks * zs);
-            ks1 = fma(ks, zc, kc * zs);
-        }
-    };
-    chunk_start(node_phase);
-    const double q0s = ks, q0s1 = ks1;
+        phase0 = (float)(-kPi);
 
-    // sums of the cosine (FP64) and sine (FP32) terms
     double sc[M];
-    float ss[M];
 #pragma unroll
     for (int j = 0; j < M; ++j)
-    {
         sc[j] = 0.0;
-        ss[j] = 0.0f;
-    }
-    auto accumulate = [&](double d, double e, double h) {
-        if constexpr (CHUNK && J0C > 0)
-            accumulate_node_chunk_c<M, J0C>(sc, ss, d, e, (float)h, zc, kc, (float)ks, kc1, (float)ks1);
-        else if constexpr (CHUNK)
-            accumulate_node_chunk<M>(sc, ss, d, e, (float)h, zc, kc, (float)ks, kc1, (float)ks1, j0d);
-        else
-            accumulate_node<M>(sc, ss, d, e, (float)h, zc, (float)zs);
-    };
-    double trap = 0.0;
-    float g_left = 0.0f;    // slope of the segment ending at the current node
-    double eps_left = 0.0;  // its width minus dphi
-    int node = 0;
+    const double j0d = (double)j0;
+    double trap = 0.0; // trig_0, the exact integral of the reference's lines
 
     const int cap = march_cap(t_near, t_far, s);
-    const float rdphi = host_reciprocal(dphi); // for the segment slopes
     // the next sample's loads are issued one step ahead (at t + s while the
     // march continues, else at t_far for the last segment)
     auto issue_at = [&](PendingSample<T, OFF32, POW2> &ps, float tt) {
@@ -435,168 +585,297 @@ __global__ __launch_bounds__(256) void generate_mixed_kernel(VolumeView<T> vol, 
     };
     PendingSample<T, OFF32, POW2> pending;
     auto density = [&](float sv) { return map_density_r<POW2>(sv, a.data_min, a.data_max, a.data_rinv); };
-    // cos and sin of the next node's phase p: those of the current node turned
-    // by dp = p - node_phase, exact in FP64 (the difference of two floats
-    // whose magnitudes are within 2^29 of each other), with sin dp and cos dp
-    // from their Taylor series to dp^5 and dp^6 (|dp| <= 2^-6: truncation
-    // below 5e-17 of sin and 1e-19 of cos); the rotation's rounding adds
-    // ~1e-16 per node. Larger steps (rays of a few dozen samples) and the
-    // march of 60 moments (whose registers are full) take the direct sincos.
-    //
-    // A chunk from J0C (compile time) turns cos and sin of j0 phi by j0 dp
-    // likewise (j0 dp rounded once), with sincos_quarter (|j0 dp| <= 50 / 64
-    // < pi / 4); otherwise, or past that step, chunk_next takes them from a
-    // sincos of j0 p.
-    constexpr bool kRotate = M <= 56;
-    bool chunk_turned = false;
-    auto advance_phase = [&](float p) {
-        const double dp = (double)p - (double)node_phase;
-        chunk_turned = false;
-        if (kRotate && fabs(dp) <= 0.015625)
+
+    // state of the node reached: its density, phase (float, as FP64) and the
+    // slope and surplus width (width - dphi) of the segment that ends there
+    double f_prev = (double)f_first, p_prev = (double)phase0;
+    double g_left = 0.0, w_left = 0.0;
+    const double dphid = (double)dphi, rdphi = 1.0 / dphid;
+    // the first increment of t and the grid's phase per unit of t
+    const float ds0 = (t + s) - t;
+    const double ptid = (double)pi_trange_inv;
+
+    issue_at(pending, fminf(t + s, t_far));
+    // advances to the next sample and to the terms of the node behind it; the
+    // last segment [p_K, 0] (src/raymarch_generate.h:107-114) starts exactly
+    // at p_K and its line ends exactly at its sample
+    float ds = ds0; // t's last increment
+    auto segment = [&](double eps, double &d, double &cp, double &cpp, double &shift) {
+        const float tn = t + s, dn = tn - t;
+        shift = 0.0;
+        if (dn != ds)
         {
-            const double d2 = dp * dp;
-            const double sd = fma(dp * d2, fma(d2, 1.0 / 120.0, -1.0 / 6.0), dp);
-            const double cd = fma(fma(fma(d2, -1.0 / 720.0, 1.0 / 24.0), d2, -0.5), d2, 1.0);
-            const double nc = fma(zc, cd, -zs * sd);
-            zs = fma(zs, cd, zc * sd);
-            zc = nc;
-            if constexpr (CHUNK && J0C > 0)
-            {
-                static_assert(J0C <= 50, "the turn by J0C dp must stay within pi / 4");
-                double sj, cj;
-                sincos_quarter((double)J0C * dp, sj, cj);
-                const double nkc = fma(kc, cj, -ks * sj);
-                ks = fma(ks, cj, kc * sj);
-                kc = nkc;
-                chunk_turned = true;
-            }
+            asm volatile(""); // rare: a branch, not a select of its result
+            shift = ((double)dn - (double)ds) * ptid;
+            ds = dn;
         }
-        else
-            sincos_small((double)p, zs, zc);
-    };
-    // cos and sin of j0 p and (j0 + 1) p at the node just reached
-    auto chunk_next = [&](float ph) {
-        if constexpr (CHUNK)
-        {
-            if (!chunk_turned)
-                sincos_small(j0d * (double)ph, ks, kc);
-            kc1 = fma(kc, zc, -ks * zs);
-            ks1 = fma(ks, zc, kc * zs);
-        }
-    };
-    issue_at(pending, (t + s < t_far) ? t + s : t_far);
-    for (int it = 0; t + s < t_far && it < cap; ++it)
-    {
-        t += s;
+        t = tn;
         const float p = (float)((double)((t - t_near) * pi_trange_inv) - kPi);
         const float f = density(pending.value());
         // the loaded values die here: keeping the next loads below this point
         // lets them land in the same registers (no copies that would wait
         // for them at the end of the iteration)
         __builtin_amdgcn_sched_barrier(0);
-        issue_at(pending, (t + s < t_far && it + 1 < cap) ? t + s : t_far);
+        issue_at(pending, fminf(t + s, t_far));
+        lo = fminf(lo, f); // f is in [0, 1]
+        hi = fmaxf(hi, f);
+        const double fd = (double)f, pd = (double)p;
+        const double u = (double)(p - dphi);
+        const double g = (fd - f_prev) * rdphi;
+        const double width = pd - u;
+        trap = fma(width, fma(0.5 * g, width, f_prev), trap);
+        const double delta = (ns > 1) ? u - p_prev : 0.0; // node 0 is the start of the first segment
+        d = g_left - g;
+        cp = fma(d, eps, -fma(g, delta, g_left * w_left));
+        cpp = f_prev * delta;
+        g_left = g;
+        w_left = width - dphid;
+        f_prev = fd;
+        p_prev = pd;
+        ++ns;
+    };
+    auto last_segment = [&](double eps, double &d, double &cp) {
+        const float f = density(pending.value());
+        lo = rmin(lo, f);
+        hi = rmax(hi, f);
+        const double dl = 0.0 - p_prev;
+        const double g = ((double)f - f_prev) / dl;
+        trap = fma(dl, fma(0.5 * g, dl, f_prev), trap);
+        d = g_left - g;
+        cp = fma(d, eps, -g_left * w_left);
+        g_left = g;
+        ++ns;
+    };
+
+    if constexpr (GRID)
+    {
+        // the phasor of the node whose weight is finished, four nodes behind,
+        // turned by the grid's step; td is that node's t
+        WeightRing ring;
+        float dsd = ds0, td = t_near;
+        double step = (double)ds0 * ptid;
+        const double rstep = 1.0 / step, rstep2 = rstep * rstep;
+        double rs, rc, zs, zc, js, jc, kr = 0.0, ki = 0.0;
+        sincos_small(step, rs, rc);
+        sincos_small(-kPi - 4.0 * step, zs, zc);
+        if constexpr (CHUNK)
+        {
+            sincos_small(j0d * step, js, jc);
+            sincos_small(j0d * (-kPi - 4.0 * step), ki, kr);
+        }
+        auto add = [&](double w) {
+            // a weight of exactly zero (inside a stretch of zero density) adds
+            // nothing; where every lane of the wavefront has one, skipped
+            if (w != 0.0)
+            {
+                if constexpr (CHUNK)
+                    accumulate_chunk<M>(sc, w, zc, kr, fma(kr, zc, -ki * zs));
+                else
+                    accumulate_blocks<M>(sc, w, zc);
+            }
+        };
+        auto turn = [&]() {
+            const double nc = fma(zc, rc, -zs * rs);
+            zs = fma(zs, rc, zc * rs);
+            zc = nc;
+            if constexpr (CHUNK)
+            {
+                const double nk = fma(kr, jc, -ki * js);
+                ki = fma(ki, jc, kr * js);
+                kr = nk;
+            }
+        };
+        // the turn to the next real node: t's increment changes where t
+        // passes a power of two
+        auto turn_real = [&]() {
+            const float tn = td + s;
+            if (tn - td != dsd)
+            {
+                dsd = tn - td;
+                sincos_small((double)dsd * ptid, rs, rc);
+                if constexpr (CHUNK)
+                    sincos_small(j0d * ((double)dsd * ptid), js, jc);
+            }
+            td = tn;
+            turn();
+        };
+        double eps = p_prev + kPi; // of node 0, at q_0 = -pi
+        int it = 0;
+        while (t + s < t_far) // t advances by s (1 - 2^-11) or more
+        {
+            double d, cp, cpp, shift;
+            segment(eps, d, cp, cpp, shift);
+            eps = p_prev - fma((double)t - (double)t_near, ptid, -kPi);
+            const double A = cpp * rstep2;
+            // where the grid's step changes by `shift` behind this node, the
+            // second difference picks up a first one
+            add(ring.push(d, A, fma(-1.2690476190476190 * A, shift, cp) * rstep));
+            if (it++ >= 4)
+                turn_real();
+            else
+                turn();
+        }
+        double d, cp;
+        last_segment(eps, d, cp);
+        add(ring.push(d, 0.0, cp * rstep));
+        // the nodes whose weights are still pending: real ones up to the
+        // last, then the grid continued
+        const int nodes = ns - 2; // index of the last node
+        for (int i = 0; i < 8; ++i)
+        {
+            if (nodes - 4 + i >= 0 && i < 4)
+                turn_real();
+            else
+                turn();
+            add(ring.pop());
+        }
+        if constexpr (!CHUNK)
+            untangle_blocks<M>(sc);
+    }
+    else
+    {
+        float ss[M];
+#pragma unroll
+        for (int j = 0; j < M; ++j)
+            ss[j] = 0.0f;
+        // cos and sin of the node phase (FP64, of the float phase); CHUNK: of
+        // j0 phi and (j0 + 1) phi too (the product j0 phi is exact in FP64)
+        float node_phase = phase0, fp = f_first, gl = 0.0f;
+        double zs, zc, kc = 1.0, ks = 0.0, kc1, ks1;
+        sincos_small((double)node_phase, zs, zc);
+        bool turned = false; // kc, ks already are those of the node
+        auto chunk_start = [&](float ph) {
+            if constexpr (CHUNK)
+            {
+                if (!turned)
+                    sincos_small(j0d * (double)ph, ks, kc);
+                kc1 = fma(kc, zc, -ks * zs);
+                ks1 = fma(ks, zc, kc * zs);
+            }
+        };
+        chunk_start(node_phase);
+        auto add = [&](double d, double e, double h) {
+            if constexpr (CHUNK && J0C > 0)
+                accumulate_node_chunk_c<M, J0C>(sc, ss, d, e, (float)h, zc, kc, (float)ks, kc1, (float)ks1);
+            else if constexpr (CHUNK)
+                accumulate_node_chunk<M>(sc, ss, d, e, (float)h, zc, kc, (float)ks, kc1, (float)ks1, j0d);
+            else
+                accumulate_node<M>(sc, ss, d, e, (float)h, zc, (float)zs);
+        };
+        const float rdphif = host_reciprocal(dphi); // for the segment slopes
+        for (int it = 0; t + s < t_far && it < cap; ++it)
+        {
+            t += s;
+            const float p = (float)((double)((t - t_near) * pi_trange_inv) - kPi);
+            const float f = density(pending.value());
+            __builtin_amdgcn_sched_barrier(0);
+            issue_at(pending, (t + s < t_far && it + 1 < cap) ? t + s : t_far);
+            ++ns;
+            lo = rmin(lo, f);
+            hi = rmax(hi, f);
+            const float u = p - dphi;
+            const float g = div_rn(f - fp, dphi, rdphif);
+            const double width = (double)p - (double)u;
+            trap += width * ((double)fp + 0.5 * (double)g * width);
+            const double delta = (it > 0) ? (double)u - (double)node_phase : 0.0;
+            const double h = fma((double)g, delta, (double)gl * w_left);
+            const double dn = (double)gl - (double)g, en = -delta * (double)fp;
+            if (dn != 0.0 || en != 0.0 || h != 0.0)
+                add(dn, en, h);
+            gl = g;
+            w_left = width - dphid;
+            fp = f;
+            // the phasor turned by the exact difference of the two float
+            // phases while that is small (Taylor terms to dp^5 and dp^6); that
+            // of j0 phi, j0 known at compile time, by j0 dp likewise
+            // (|j0 dp| <= 50 / 64 < pi / 4)
+            const double dp = (double)p - (double)node_phase;
+            turned = false;
+            if (M <= 56 && fabs(dp) <= 0.015625)
+            {
+                const double d2 = dp * dp;
+                const double sd = fma(dp * d2, fma(d2, 1.0 / 120.0, -1.0 / 6.0), dp);
+                const double cd = fma(fma(fma(d2, -1.0 / 720.0, 1.0 / 24.0), d2, -0.5), d2, 1.0);
+                const double nc = fma(zc, cd, -zs * sd);
+                zs = fma(zs, cd, zc * sd);
+                zc = nc;
+                if constexpr (CHUNK && J0C > 0)
+                {
+                    static_assert(J0C <= 50, "the turn by J0C dp must stay within pi / 4");
+                    double sj, cj;
+                    sincos_quarter((double)J0C * dp, sj, cj);
+                    const double nkc = fma(kc, cj, -ks * sj);
+                    ks = fma(ks, cj, kc * sj);
+                    kc = nkc;
+                    turned = true;
+                }
+            }
+            else
+                sincos_small((double)p, zs, zc);
+            node_phase = p;
+            chunk_start(p);
+        }
+        // last segment [p_K, 0] (src/raymarch_generate.h:107-114): it starts
+        // exactly at p_K and its line ends exactly at its sample
+        const float f = density(pending.value());
         ++ns;
         lo = rmin(lo, f);
         hi = rmax(hi, f);
-        // the reference's segment [u, p]: u = p - dphi in float, slope (f - f_prev) / dphi
-        const float u = p - dphi;
-        const float g = div_rn(f - f_prev, dphi, rdphi);
-        const double width = (double)p - (double)u;
-        trap += width * ((double)f_prev + 0.5 * (double)g * width);
-        // the offset of the segment start from the node (exact: u and the
-        // node phase are floats a few ulps apart) and the terms of the node
-        const double delta = (node > 0) ? (double)u - (double)node_phase : 0.0;
-        const double h = fma((double)g, delta, (double)g_left * eps_left);
-        // a node with d = e = h = 0 (inside a stretch of zero density:
-        // both slopes and the start value vanish) adds exact zeros; where
-        // every lane of the wavefront has one, the update is skipped
-        {
-            const double dn = (double)g_left - (double)g, en = -delta * (double)f_prev;
-            if (dn != 0.0 || en != 0.0 || h != 0.0)
-                accumulate(dn, en, h);
-        }
-        g_left = g;
-        eps_left = width - (double)dphi;
-        f_prev = f;
-        advance_phase(p);
-        node_phase = p;
-        ++node;
-        chunk_next(p);
+        const float dl = 0.0f - node_phase;
+        const float g = (f - fp) / dl;
+        trap += (double)dl * ((double)fp + 0.5 * (double)g * (double)dl);
+        add((double)gl - (double)g, 0.0, (double)gl * w_left);
+        g_left = (double)g;
+#pragma unroll
+        for (int j = 0; j < M; ++j)
+            sc[j] = fma(j0d + (double)j, (double)ss[j], sc[j]);
     }
-    // last segment [p_K, 0] (src/raymarch_generate.h:107-114): it starts
-    // exactly at p_K and its line ends exactly at f_last
-    const float f_last = density(pending.value());
-    ++ns;
-    lo = rmin(lo, f_last);
-    hi = rmax(hi, f_last);
-    const float dl = 0.0f - node_phase;
-    const float g_last = (f_last - f_prev) / dl;
-    trap += (double)dl * ((double)f_prev + 0.5 * (double)g_last * (double)dl);
-    accumulate((double)g_left - (double)g_last, 0.0, (double)g_left * eps_left);
     // node at phase 0: cos(j*0) = 1, sin(j*0) = 0
 #pragma unroll
     for (int j = CHUNK ? 0 : 1; j < M; ++j)
-        sc[j] += (double)g_last;
+        sc[j] += g_left;
 
-    // trig_j = (sc_j + j ss_j) / j^2 - f_0 sin(j phi_0) / j in FP64, sin by
-    // Chebyshev from phi_0 (from j0 phi_0 and (j0 + 1) phi_0 for a chunk),
-    // then moment_j = trig_j / pi, normalised and rounded to float once
-    double trig[M];
-    {
-        const double x2 = z0c + z0c;
-        double sm2 = CHUNK ? q0s : 0.0, sm1 = CHUNK ? q0s1 : z0s;
-#pragma unroll
-        for (int i = CHUNK ? 0 : 1; i < M; ++i)
-        {
-            double sj;
-            if (CHUNK && i == 0)
-                sj = q0s;
-            else if (i == 1)
-                sj = CHUNK ? q0s1 : z0s;
-            else
-            {
-                sj = fma(x2, sm1, -sm2);
-                sm2 = sm1;
-                sm1 = sj;
-            }
-            const double jd = j0d + (double)i;
-            const double num = fma(jd, (double)ss[i], sc[i]);
-            trig[i] = (jd == 0.0) ? 0.0 : num / (jd * jd) - (double)f_first * sj / jd;
-        }
-    }
-    if (first_chunk)
-        trig[0] = trap;
-
-    uint32_t b;
-    constexpr double kInvPi = 0.31830988618379067154;
+    // trig_j = sc_j / j^2 - f_0 sin(j phi_0) / j in FP64 (phi_0 the start of
+    // the first segment), sin by the recurrence over j, then moment_j =
+    // trig_j / pi, normalised and rounded to float once
+    double norm = 0.31830988618379067154; // 1 / pi
     if (a.transform_to_bounds)
     {
         lo = rmax(lo - a.bound_eps, 0.0f);
         hi = rmin(hi + a.bound_eps, 1.0f);
         const double inv = 1.0 / (double)(hi - lo);
         if (first_chunk)
-            mo[0] = (float)((trig[0] * kInvPi - (double)lo) * inv);
-#pragma unroll
-        for (int i = 0; i < M; ++i)
-        {
-            const int j = j0 + i;
-            if (j >= 1 && j < jend)
-                mo[j] = (float)(trig[i] * kInvPi * inv);
-        }
+            mo[0] = (float)((trap * norm - (double)lo) * inv);
+        norm *= inv;
     }
-    else
+    else if (first_chunk)
+        mo[0] = (float)(trap * norm);
     {
+        double z0s, z0c, k0s = 0.0, k0c = 1.0;
+        sincos_small((double)phase0, z0s, z0c);
+        if constexpr (CHUNK)
+            sincos_small(j0d * (double)phase0, k0s, k0c);
+        const double x2 = z0c + z0c;
+        double sm2 = k0s, sm1 = fma(k0s, z0c, k0c * z0s); // sin(j0 phi_0), sin((j0 + 1) phi_0)
 #pragma unroll
         for (int i = 0; i < M; ++i)
         {
+            const double jd = j0d + (double)i;
             const int j = j0 + i;
-            if (j < jend)
-                mo[j] = (float)(trig[i] * kInvPi);
+            double sj = (i == 0) ? sm2 : sm1;
+            if (i >= 1)
+            {
+                const double n = fma(x2, sm1, -sm2);
+                sm2 = sm1;
+                sm1 = n;
+            }
+            if (j >= 1 && j < jend)
+                mo[j] = (float)((sc[i] / (jd * jd) - (double)f_first * sj / jd) * norm);
         }
     }
     if (first_chunk)
     {
-        b = pack_bound(lo, hi);
+        const uint32_t b = pack_bound(lo, hi);
         if (bounds)
             bounds[pix] = b;
         if (ray_range)
@@ -610,12 +889,11 @@ __global__ __launch_bounds__(256) void generate_mixed_kernel(VolumeView<T> vol, 
 // launchers
 // ---------------------------------------------------------------------------
 // one launch of generate_mixed_kernel over `chunks` rows of blockIdx.y
-template <typename T, int M, bool CHUNK, int J0C>
+template <typename T, int M, bool CHUNK, bool GRID, int J0C>
 static void launch_mixed_kernel(const VolumeView<T> &v, const DevCamera &c, const GenArgs &a, float *o, uint32_t *b,
                                 int32_t *s, float2 *rr, hipStream_t st, uint32_t blocks, int chunks)
 {
-    // byte offsets of every voxel fit in 32 bits up to 4 GiB of volume
-    const bool off32 = (uint64_t)v.nx * v.ny * v.nz * sizeof(T) <= (uint64_t)0xFFFFFFFFu + 1u;
+    const bool off32 = offsets_fit(v.nx, v.ny, v.nz, sizeof(T));
     // power-of-two domain extents and data range: divisions become products
     const bool pow2 = exact_pow2(v.dmax.x - v.dmin.x) && exact_pow2(v.dmax.y - v.dmin.y) &&
                       exact_pow2(v.dmax.z - v.dmin.z) && exact_pow2(a.data_max - a.data_min);
@@ -624,49 +902,49 @@ static void launch_mixed_kernel(const VolumeView<T> &v, const DevCamera &c, cons
     {
         // particle sets: the gather ignores OFF32 and POW2 (the data range
         // division takes the exact path)
-        hipLaunchKernelGGL((generate_mixed_kernel<T, M, true, false, CHUNK, J0C>), grid, dim3(256), 0, st, v, c, a,
+        hipLaunchKernelGGL((generate_mixed_kernel<T, M, true, false, CHUNK, GRID, J0C>), grid, dim3(256), 0, st, v, c, a,
                            o, b, s, rr);
     }
     else
     {
         if (off32 && pow2)
-            hipLaunchKernelGGL((generate_mixed_kernel<T, M, true, true, CHUNK, J0C>), grid, dim3(256), 0, st, v, c, a,
-                               o, b, s, rr);
+            hipLaunchKernelGGL((generate_mixed_kernel<T, M, true, true, CHUNK, GRID, J0C>), grid, dim3(256), 0, st, v, c,
+                               a, o, b, s, rr);
         else if (off32)
-            hipLaunchKernelGGL((generate_mixed_kernel<T, M, true, false, CHUNK, J0C>), grid, dim3(256), 0, st, v, c,
+            hipLaunchKernelGGL((generate_mixed_kernel<T, M, true, false, CHUNK, GRID, J0C>), grid, dim3(256), 0, st, v, c,
                                a, o, b, s, rr);
         else
-            hipLaunchKernelGGL((generate_mixed_kernel<T, M, false, false, CHUNK, J0C>), grid, dim3(256), 0, st, v, c,
-                               a, o, b, s, rr);
+            hipLaunchKernelGGL((generate_mixed_kernel<T, M, false, false, CHUNK, GRID, J0C>), grid, dim3(256), 0, st, v,
+                               c, a, o, b, s, rr);
     }
 }
 
-// CHUNK marches the moments in chunks of M: the unchunked kernel for the
-// first, then the second from j0 = M as a compile-time start, or the later
-// ones over blockIdx.y
-template <typename T, int M, bool CHUNK = false>
+// `chunks` > 1 marches the moments in chunks of M: the unchunked kernel for
+// the first, then the later ones over blockIdx.y (or, summed node by node and
+// two, the second from j0 = M as a compile-time start)
+template <typename T, int M, bool GRID, bool CHUNK = false>
 static void launch_mixed(const VolumeView<T> &v, const DevCamera &c, const GenArgs &a, float *o, uint32_t *b,
                          int32_t *s, float2 *rr, hipStream_t st, uint32_t blocks, int chunks = 1)
 {
-    launch_mixed_kernel<T, M, false, 0>(v, c, a, o, b, s, rr, st, blocks, 1);
+    launch_mixed_kernel<T, M, false, GRID, 0>(v, c, a, o, b, s, rr, st, blocks, 1);
     if constexpr (CHUNK)
     {
-        if (chunks == 2)
-            launch_mixed_kernel<T, M, true, M>(v, c, a, o, b, s, rr, st, blocks, 1);
-        else if (chunks > 2)
-            launch_mixed_kernel<T, M, true, 0>(v, c, a, o, b, s, rr, st, blocks, chunks - 1);
+        if (chunks == 2 && !GRID)
+            launch_mixed_kernel<T, M, true, GRID, GRID ? 0 : M>(v, c, a, o, b, s, rr, st, blocks, 1);
+        else if (chunks > 1)
+            launch_mixed_kernel<T, M, true, GRID, 0>(v, c, a, o, b, s, rr, st, blocks, chunks - 1);
     }
 }
 
-template <typename T>
-static int dispatch_mixed(const VolumeView<T> &v, const DevCamera &c, const GenArgs &a, float *o, uint32_t *b,
-                          int32_t *s, float2 *rr, hipStream_t st, uint32_t blocks)
+template <typename T, bool GRID>
+static int dispatch_widths(const VolumeView<T> &v, const DevCamera &c, const GenArgs &a, float *o, uint32_t *b,
+                           int32_t *s, float2 *rr, hipStream_t st, uint32_t blocks)
 {
     const int m = a.m;
 #define MRAY_GEN_CASE(MM)                                                                                             \
     if (m <= MM)                                                                                                      \
     {                                                                                                                 \
-        launch_mixed<T, MM>(v, c, a, o, b, s, rr, st, blocks);                                                            \
+        launch_mixed<T, MM, GRID>(v, c, a, o, b, s, rr, st, blocks);                                                  \
         return 0;                                                                                                     \
     }
     MRAY_GEN_CASE(4)
@@ -693,17 +971,58 @@ static int dispatch_mixed(const VolumeView<T> &v, const DevCamera &c, const GenA
     {
         const int chunks = (m + 49) / 50;
         const int per = (m + chunks - 1) / chunks;
-#define MRAY_GEN_CHUNK_CASE(MM)                                                                                       \
-    if (per <= MM)                                                                                                    \
-    {                                                                                                                 \
-        launch_mixed<T, MM, true>(v, c, a, o, b, s, rr, st, blocks, chunks);                                          \
-        return 0;                                                                                                     \
-    }
-        MRAY_GEN_CHUNK_CASE(40)
-        MRAY_GEN_CHUNK_CASE(50)
-#undef MRAY_GEN_CHUNK_CASE
+        if (per <= 40)
+            launch_mixed<T, 40, GRID, true>(v, c, a, o, b, s, rr, st, blocks, chunks);
+        else
+            launch_mixed<T, 50, GRID, true>(v, c, a, o, b, s, rr, st, blocks, chunks);
+        return 0;
     }
     return MRAY_ERR_UNSUPPORTED;
+}
+
+// The gridded march for the wavefronts whose rays the grid resolves, the march
+// summed node by node for the others: both launches, unless one is known to
+// have no wavefront. A pass that records the rays' normalisation (ray_range)
+// is summed node by node throughout (see the kernel), and so is an image whose
+// longest possible ray has too few samples for its moments; all rays of an
+// orthographic camera along an axis are as long as the box.
+template <typename T>
+static int dispatch_mixed(const VolumeView<T> &v, const DevCamera &c, const GenArgs &a, float *o, uint32_t *b,
+                          int32_t *s, float2 *rr, hipStream_t st, uint32_t blocks)
+{
+    GenArgs g = a;
+    const float ex = v.dmax.x - v.dmin.x, ey = v.dmax.y - v.dmin.y, ez = v.dmax.z - v.dmin.z;
+    const Vec3 d = c.dir;
+    // directions of perspective rays are unit vectors, an orthographic
+    // camera's is as given
+    const float len = c.orthographic ? sqrtf(d.x * d.x + d.y * d.y + d.z * d.z) : 1.0f;
+    const float longest = sqrtf(ex * ex + ey * ey + ez * ez) / len;
+    g.rays = kRaysAll;
+    if (rr || !((float)(a.m - 1) * (float)kPi * (a.step / longest) <= 1.01f))
+        return dispatch_widths<T, false>(v, c, g, o, b, s, rr, st, blocks);
+    const int rc = dispatch_widths<T, true>(v, c, g, o, b, s, rr, st, blocks);
+    if (rc != 0)
+        return rc;
+    const int axes = (d.x != 0.0f) + (d.y != 0.0f) + (d.z != 0.0f);
+    if (c.orthographic && axes == 1)
+    {
+        const float along = (d.x != 0.0f ? ex : d.y != 0.0f ? ey : ez) / len;
+        // from outside the box (znear cuts nothing off), with a margin for
+        // rounding, and not too many steps from the camera
+        const float from = d.x != 0.0f ? (d.x > 0 ? v.dmin.x - c.pos.x : c.pos.x - v.dmax.x)
+                           : d.y != 0.0f ? (d.y > 0 ? v.dmin.y - c.pos.y : c.pos.y - v.dmax.y)
+                                         : (d.z > 0 ? v.dmin.z - c.pos.z : c.pos.z - v.dmax.z);
+        // the slab's near end is at from / len for every pixel (right and up
+        // have no component along the axis)
+        const float ru = d.x != 0.0f ? fabsf(c.right.x) + fabsf(c.up.x)
+                         : d.y != 0.0f ? fabsf(c.right.y) + fabsf(c.up.y)
+                                       : fabsf(c.right.z) + fabsf(c.up.z);
+        if (ru == 0.0f && from / len > c.znear && (float)(a.m - 1) * (float)kPi * (a.step / along) <= 0.99f &&
+            (from / len + along) * 1.01f <= 8192.0f * a.step && a.step < 0.5f * along)
+            return 0;
+    }
+    g.rays = kRaysUngridded;
+    return dispatch_widths<T, false>(v, c, g, o, b, s, rr, st, blocks);
 }
 
 // PLAIN keeps m floats per thread in LDS: 256-thread blocks while that fits
@@ -1304,6 +1623,7 @@ int launch_generate_adjoint(const float *vox, int nx, int ny, int nz, const floa
     a.transform_to_bounds = p.transform_to_bounds;
     a.compact_image = p.compact_image;
     a.bound_eps = p.transform_bound_eps;
+    a.rays = kRaysAll;
     DevCamera c = make_dev_camera(cam);
     const uint32_t ntiles = (uint32_t)(((W + 7) / 8) * ((H + 7) / 8));
     const uint32_t blocks = (ntiles + 3) / 4;
@@ -1377,6 +1697,7 @@ int launch_generate(const void *vox, int dtype, int nx, int ny, int nz, const fl
     a.transform_to_bounds = p.transform_to_bounds;
     a.compact_image = p.compact_image;
     a.bound_eps = p.transform_bound_eps;
+    a.rays = kRaysAll;
     DevCamera c = make_dev_camera(cam);
     uint32_t ntiles = (uint32_t)(((W + 7) / 8) * ((H + 7) / 8));
     uint32_t blocks = (ntiles + 3) / 4;

@@ -111,7 +111,7 @@ int launch_typed(const T *vox, int nx, int ny, int nz, const float *dmin, const 
     const uint32_t ntiles = (uint32_t)(((a.W + 7) / 8) * ((a.H + 7) / 8));
     const dim3 grid((ntiles + 3) / 4);
     // byte offsets of every voxel fit in 32 bits up to 4 GiB of volume
-    const bool off32 = (uint64_t)nx * ny * nz * sizeof(T) <= (uint64_t)0xFFFFFFFFu + 1u;
+    const bool off32 = offsets_fit(nx, ny, nz, sizeof(T));
     if (off32)
         hipLaunchKernelGGL((reference_kernel<T, true>), grid, dim3(256), 0, stream, v, c, a, tf, rgba, steps);
     else

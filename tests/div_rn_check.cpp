@@ -1,7 +1,7 @@
 // Check of mray::div_rn_core (mray_amd/csrc/div_rn.hpp) against IEEE float
 // division: for each divisor significand below, every dividend significand
 // in [1, 2) and the quotient are compared bit for bit. Built and run by
-// tests/test_division.py. Prints "<pairs> <mismatches> <fast-path rejects> <range guards ok>".
+// tests/test_division.py. Prints "<pairs> <mismatches> <fast-path rejects> <range guards ok> <keys ok> <exact bytes>".
 #include <cstdio>
 #include <cstdlib>
 #include <cstring>
@@ -63,6 +63,14 @@ int main(int argc, char **argv)
     const float big = mray::host_reciprocal(0x1p31f), tiny = mray::host_reciprocal(0x1p-31f);
     const int guards = (big != big) && (tiny != tiny) && !mray::div_rn_fast_ok(1.0f, mray::div_rn_core(1.0f, 0x1p31f, big)) &&
                        !mray::div_rn_fast_ok(0.0f, 0.0f) && !mray::div_rn_fast_ok(-0.0f, 0.0f);
-    printf("%ld %ld %ld %d\n", pairs, bad, rejected, guards);
+    // dividends checked together: zero and 2^-60 pass, the next magnitude below does not
+    const int keys = mray::div_rn_key(0.0f) >= mray::kDivRnKeyMin && mray::div_rn_key(-0.0f) >= mray::kDivRnKeyMin &&
+                     mray::div_rn_key(-0x1p-60f) >= mray::kDivRnKeyMin && mray::div_rn_key(1.0f) >= mray::kDivRnKeyMin &&
+                     mray::div_rn_key(0x1.fffffep-61f) < mray::kDivRnKeyMin &&
+                     mray::div_rn_key(-0x1p-140f) < mray::kDivRnKeyMin && mray::div_rn_core(0.0f, 3.0f, mray::host_reciprocal(3.0f)) == 0.0f;
+    int bytes = 0;
+    for (int v = 0; v < 256; ++v)
+        bytes += mray::byte_unit((uint8_t)v) == (float)(v / 255.f);
+    printf("%ld %ld %ld %d %d %d\n", pairs, bad, rejected, guards, keys, bytes);
     return 0;
 }

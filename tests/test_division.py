@@ -26,9 +26,10 @@ def test_div_rn_matches_ieee_division(tmp_path):
     subprocess.run(["g++", "-O2", "-fopenmp", "-ffp-contract=off", "-o", str(exe),
                     str(HERE / "div_rn_check.cpp")], check=True)
     out = subprocess.run([str(exe), "64"], check=True, capture_output=True, text=True, timeout=600).stdout.split()
-    pairs, bad, rejected, guards = map(int, out)
+    pairs, bad, rejected, guards, keys, exact_bytes = map(int, out)
     assert pairs == (64 + 64) * 3 * (1 << 23)
     assert bad == 0, f"{bad} quotients differ from IEEE division"
     assert rejected == 0, "in-range operands must take the three-operation path"
     assert guards == 1, "divisors outside [2^-30, 2^30] and zero dividends must take the IEEE division"
-
+    assert keys == 1, "the joint range check must pass zero and 2^-60 and refuse smaller dividends"
+    assert exact_bytes == 256, "a byte voxel's value must be the IEEE quotient v / 255"

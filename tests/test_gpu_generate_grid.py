@@ -1,0 +1,58 @@
+"""The gridded march of generate against the march summed node by node.
+
+A call that records the rays' normalisation (ray_range) sums every ray's
+moments node by node; without it, the rays whose samples resolve the largest
+order take the gridded march. Both evaluate the same integral in FP64 and round
+each moment to float once: per ray they may differ by one rounding of the
+largest moment (2^-23 of it; the gridded stencils add up to 1e-9, the node sums
+up to 3e-8 on their own FP32 terms). Bounds and sample counts are the same bits.
+Sizes: orders from far below to just past what the samples resolve, chunks of
+moments, images that are no multiple of a tile, t that passes powers of two
+(whose increments change there), more than 8192 steps from the camera, and
+domains that are no power of two in byte and float volumes."""
+import numpy as np
+import pytest
+import torch
+
+pytestmark = pytest.mark.gpu
+
+from mray_amd import hip, synth  # noqa: E402
+from mray_amd.types import GenParams  # noqa: E402
+
+CASES = {
+    # n, (dmin, dmax), camera, W, H, m, step
+    "resolved": (64, (-1, 1), synth.ortho_camera(), 24, 17, 20, 1.0 / 64),
+    "limit": (64, (-1, 1), synth.ortho_camera(), 16, 16, 41, 1.0 / 64),
+    "past_limit": (64, (-1, 1), synth.ortho_camera(), 16, 16, 42, 1.0 / 64),
+    "persp_mixed": (48, (0, 1), synth.perspective_camera(aspect=40 / 30), 40, 30, 24, 0.5 / 48),
+    "chunks2": (96, (0, 1), synth.perspective_camera(position=(0.45, 0.5, -0.9)), 19, 21, 61, 0.25 / 96),
+    "chunks3": (96, (0, 1), synth.perspective_camera(), 16, 9, 101, 0.15 / 96),
+    "increments": (80, (0, 1), synth.perspective_camera(position=(0.5, 0.5, -3.3), fov_half_deg=9.0), 24, 24, 33,
+                   0.37 / 80),
+    "far": (32, (0, 1), synth.perspective_camera(position=(0.5, 0.5, -90.0), fov_half_deg=0.3), 8, 8, 16, 0.01),
+    "oblong": (50, (0, 0.9375), synth.perspective_camera(position=(0.4, 0.5, -1.0)), 24, 24, 30, 0.5 / 50),
+    "one": (32, (0, 1), synth.perspective_camera(), 9, 9, 1, 0.5 / 32),
+    "two": (32, (0, 1), synth.perspective_camera(), 9, 9, 2, 0.5 / 32),
+}
+
+
+@pytest.mark.parametrize("dtype", ["f32", "u8"])
+@pytest.mark.parametrize("name", list(CASES))
+def test_gridded_march_matches_node_sums(name, dtype):
+    n, (lo, hi), cam, W, H, m, step = CASES[name]
+    vol = synth.marschner_lobb(n) if lo < 0 else synth.mixing_layer(n, width=0.05)
+    v = torch.from_numpy(vol).cuda()
+    if dtype == "u8":
+        v = (v.clamp(0, 1) * 255).to(torch.uint8)
+    vol = hip.Volume(v, (lo,) * 3, (hi,) * 3)
+    gp = GenParams(step_size=step, transform_to_bounds=1, transform_bound_eps=0.01, compact_image=0,
+                   prediction_coding=0, bias=1e-4)
+    rr = torch.empty((H * W, 2), dtype=torch.float32, device="cuda")
+    ref, b_ref, s_ref = hip.generate(vol, cam, gp, W, H, m, ray_range=rr, want_samples=True)
+    mo, b, s = hip.generate(vol, cam, gp, W, H, m, want_samples=True)
+    assert torch.equal(b, b_ref) and torch.equal(s, s_ref)
+    d = (mo.double() - ref.double()).view(-1, m).abs().amax(1)
+    size = ref.double().view(-1, m).abs().amax(1)
+    assert bool((size > 0).any())
+    bound = 2.0 ** -23 * size + 4e-8
+    assert bool((d <= bound).all()), f"{name}: {float((d / bound).max()):.2f} of the bound"
