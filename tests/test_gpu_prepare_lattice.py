@@ -1,0 +1,89 @@
+"""The MIXED preparation's lattice kernels against the FP64 oracle
+(orc_prepare_moments_std_f64: Levinson's recursion, in FP64).
+
+Both solve the same Toeplitz system in FP64, so at MESE bias 1e-3 and these
+densities (|u|^2 up to ~0.99) multipliers agree to a small multiple of the
+conditioning times 2^-53; the bound is 1e-9 of a pixel's largest multiplier
+(f32 multipliers: half an ulp more). Counts at the edges of the lanes' blocks
+(4, 8 and 16 lanes per pixel, by image size and by moments), compact images of
+ragged counts with empty pixels, and moments outside the moment space, where
+the |u|^2 >= 1 guard fires and every later coefficient is 0."""
+import numpy as np
+import pytest
+import torch
+
+pytestmark = pytest.mark.gpu
+
+from mray_amd import hip  # noqa: E402
+from oracle_ffi import Oracle  # noqa: E402
+
+
+@pytest.fixture(scope="module")
+def O():
+    hip.init(0)
+    return Oracle()
+
+
+def densities(rng, n, m):
+    """Moments of random piecewise-constant densities in [0.03, 0.97], f32."""
+    cut = np.sort(rng.uniform(-np.pi, 0, (n, 4)), axis=1)
+    phi = np.concatenate([np.full((n, 1), -np.pi), cut, np.zeros((n, 1))], axis=1)
+    val = rng.uniform(0.03, 0.97, (n, 5))
+    mo = np.empty((n, m))
+    mo[:, 0] = ((phi[:, 1:] - phi[:, :-1]) * val).sum(1) / np.pi
+    for j in range(1, m):
+        s = np.sin(j * phi)
+        mo[:, j] = ((s[:, 1:] - s[:, :-1]) * val).sum(1) / (np.pi * j) * np.exp(-0.5 * (0.05 * j) ** 2)
+    return mo.astype(np.float32)
+
+
+def check(O, mo, lag, nm, bias, tol):
+    for i in range(len(nm)):
+        ref = O.prepare_std_f64(int(nm[i]), mo[i][:nm[i]].astype(np.float64), float(np.float32(bias)))
+        assert np.abs(lag[i][:nm[i]] - ref).max() <= tol * np.abs(ref).max(), (i, nm[i])
+
+
+# images of up to 4096, up to 8192 and more pixels take 16, 8 and 4 lanes
+@pytest.mark.parametrize("W,H", [(9, 7), (64, 64), (65, 64), (128, 64), (129, 64)])
+@pytest.mark.parametrize("m", [1, 2, 7, 8, 9, 31, 33, 50, 100, 101, 129, 193, 255])
+def test_dense(O, W, H, m):
+    if W * H > 100 and m not in (8, 33, 50, 100, 101):
+        pytest.skip("edges of the lane blocks are covered at the smallest size")
+    rng = np.random.default_rng(W * 1000 + m)
+    mo = densities(rng, W * H, m)
+    lag = hip.prepare(torch.from_numpy(mo).cuda(), W, H, m, 1e-3, form="mixed64").cpu().numpy().reshape(-1, m)
+    pick = np.unique(np.concatenate([np.arange(3), rng.integers(0, W * H, 12), np.arange(W * H - 3, W * H)]))
+    check(O, mo[pick], lag[pick], np.full(len(pick), m), 1e-3, 1e-9)
+    f32 = hip.prepare(torch.from_numpy(mo).cuda(), W, H, m, 1e-3, form="mixed").cpu().numpy().reshape(-1, m)
+    assert np.array_equal(f32, lag.astype(np.float32))
+
+
+@pytest.mark.parametrize("W,H", [(12, 11), (70, 70), (130, 64)])
+def test_compact_ragged(O, W, H):
+    m = 60
+    rng = np.random.default_rng(W)
+    mo = densities(rng, W * H, m)
+    nm = rng.integers(0, m + 1, W * H)
+    nm[:40] = np.arange(40) % (m + 1)
+    nm[-3:] = (0, 1, m)
+    index = np.concatenate([[0], np.cumsum(nm)]).astype(np.int32)
+    data = np.concatenate([mo[i][:nm[i]] for i in range(W * H)])
+    lag = hip.prepare(torch.from_numpy(data).cuda(), W, H, m, 1e-3, form="mixed64",
+                      index=torch.from_numpy(index).cuda()).cpu().numpy()
+    pick = np.unique(np.concatenate([np.arange(48), rng.integers(0, W * H, 40), np.arange(W * H - 3, W * H)]))
+    pick = pick[nm[pick] > 0]
+    check(O, mo[pick], [lag[index[i]:index[i + 1]] for i in pick], nm[pick], 1e-3, 1e-9)
+
+
+@pytest.mark.parametrize("W,H", [(8, 8), (80, 64), (130, 64)])
+def test_outside_the_moment_space(O, W, H):
+    """A valid prefix, then a jump that no density has: the guard fires there in
+    every implementation (|u| far above 1), the later coefficients are 0."""
+    m = 24
+    rng = np.random.default_rng(5)
+    mo = densities(rng, W * H, m)
+    mo[:, 12] += 3.0
+    mo[::3, 5] -= 2.0
+    lag = hip.prepare(torch.from_numpy(mo).cuda(), W, H, m, 1e-3, form="mixed64").cpu().numpy().reshape(-1, m)
+    pick = rng.integers(0, W * H, 30)
+    check(O, mo[pick], lag[pick], np.full(30, m), 1e-3, 1e-9)
