@@ -22,7 +22,7 @@
 //         Two marches sum these terms. Where the samples resolve the largest
 //         order (almost every ray), the ulp-sized terms become weights of
 //         plain cosines on the ray's uniform phase grid (WeightRing), and a
-//         moment costs one FP64 operation per node (accumulate_blocks); the
+//         moment costs one FP64 operation per node (block_sums); the
 //         other rays are summed node by node from each node's own phasor,
 //         five operations per moment (accumulate_node). gfx950 issues FP64
 //         FMAs at the rate of unpacked FP32 ones, so the cosine sums and
@@ -30,6 +30,7 @@
 //         moments are rounded to float once. Moments live in registers
 //         (template M >= m); more than 60 are split into chunks over
 //         workgroups (CHUNK).
+#include "cheb_blocks.hpp"
 #include "device_common.hpp"
 #include "launch.hpp"
 #include "sph_common.hpp"
@@ -194,68 +195,6 @@ __global__ __launch_bounds__(256) void generate_plain_kernel(VolumeView<T> vol, 
 // ---------------------------------------------------------------------------
 // MIXED
 // ---------------------------------------------------------------------------
-
-// The moment sums of a march keep, for every node n of the ray's uniform
-// phase grid q_n, one weight w_n (the stencil below): sc_j = sum_n w_n
-// cos(j q_n), trig_j = sc_j / j^2 up to the ray's first sample. In FP64:
-// gfx950 issues FP64 FMAs at the rate of unpacked FP32 ones.
-//
-// accumulate_blocks takes the cosines as products, j = q P + r:
-//     a_qr += (w T_qP(x)) T_r(x),   x = cos(q_n),
-// with T_r, r < P, and w T_qP by their Chebyshev recurrences, so that a
-// moment costs one operation and a node P + M / P more, instead of two per
-// moment. 2 T_qP T_r = T_qP+r + T_qP-r, so the sums of cosines follow from the
-// sums of products once per ray (untangle_blocks). P near sqrt(M) makes the
-// overhead smallest; slot 0 (moment 0, integrated separately) is not summed.
-template <int M> constexpr int block_width() { return M <= 12 ? 4 : M <= 30 ? 5 : M <= 56 ? 7 : M <= 72 ? 8 : 10; }
-
-template <int M> __device__ __forceinline__ void accumulate_blocks(double (&sc)[M], double w, double x)
-{
-    constexpr int P = block_width<M>();
-    const double x2 = x + x;
-    double T[P + 1];
-    T[0] = 1.0;
-    T[1] = x;
-#pragma unroll
-    for (int r = 2; r <= P; ++r)
-        T[r] = fma(x2, T[r - 1], -T[r - 2]);
-    const double y2 = T[P] + T[P];
-    double z1 = w, z = w;
-#pragma unroll
-    for (int q = 0; q * P < M; ++q)
-    {
-        if (q == 1)
-            z = w * T[P];
-        else if (q > 1)
-        {
-            const double zn = fma(y2, z, -z1);
-            z1 = z;
-            z = zn;
-        }
-#pragma unroll
-        for (int r = 0; r < P; ++r)
-        {
-            const int j = q * P + r;
-            if (j >= M || j == 0)
-                continue;
-            if (r == 0)
-                sc[j] += z;
-            else
-                sc[j] = fma(z, T[r], sc[j]);
-        }
-    }
-}
-
-// sums of cosines from accumulate_blocks' sums of products:
-// sc_qP+r = 2 a_qr - sc_qP-r for q, r >= 1 (the other slots are products with T_0)
-template <int M> __device__ __forceinline__ void untangle_blocks(double (&sc)[M])
-{
-    constexpr int P = block_width<M>();
-#pragma unroll
-    for (int j = P + 1; j < M; ++j)
-        if (j % P != 0)
-            sc[j] = fma(2.0, sc[j], -sc[j / P * P - j % P]);
-}
 
 // The chunk j0 .. j0 + M - 1 of a march whose moments are split into chunks:
 // sc_i += w cos((j0 + i) q_n) by the recurrence from w cos(j0 q_n) and
@@ -671,7 +610,12 @@ __global__ __launch_bounds__(256, 2) void generate_mixed_kernel(VolumeView<T> vo
                 if constexpr (CHUNK)
                     accumulate_chunk<M>(sc, w, zc, kr, fma(kr, zc, -ki * zs));
                 else
-                    accumulate_blocks<M>(sc, w, zc);
+                {
+                    // moment 0 is integrated apart (trap)
+                    double cheb[block_width<M>() + 1];
+                    cheb_low<block_width<M>()>(cheb, zc);
+                    block_sums<M, 1>(sc, w, cheb);
+                }
             }
         };
         auto turn = [&]() {
@@ -730,7 +674,7 @@ __global__ __launch_bounds__(256, 2) void generate_mixed_kernel(VolumeView<T> vo
             add(ring.pop());
         }
         if constexpr (!CHUNK)
-            untangle_blocks<M>(sc);
+            untangle_sums<M>(sc);
     }
     else
     {

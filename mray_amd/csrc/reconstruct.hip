@@ -21,8 +21,10 @@
 //         cancellation, while FP64 FMAs cost the same issue slots as FP32
 //         ones on gfx950. The 256-entry transfer function is staged in LDS
 //         once per workgroup.
+#include "cheb_blocks.hpp"
 #include "device_common.hpp"
 #include "launch.hpp"
+#include <type_traits>
 
 namespace mray
 {
@@ -194,50 +196,16 @@ __device__ __forceinline__ double cos_theta_of(float p)
     return reflect ? q2 - 1.0 : 1.0 - q2;
 }
 
-template <int M, typename L>
-__device__ __forceinline__ double series_clenshaw(const L (&lam)[M], float p, double *cos_theta = nullptr)
+// lambda_0 + 2 sum_{l=1}^{M-1} lambda_l cos(l theta), theta = -p in [0, pi],
+// from the products' coefficients of (lambda_0, 2 lambda_l) (entries l >= m
+// hold 0); x = cos(theta) and T_r of it are left to the caller. FP64: gfx950
+// issues FP64 FMAs at the non-packed FP32 rate. At 50 moments 64 operations
+// (98 by Clenshaw's recurrence over the orders).
+template <int M>
+__device__ __forceinline__ double series_at(const double (&c)[M], float p, double (&T)[block_width<M>() + 1])
 {
-    // lambda_0 + 2 sum_{l=1}^{M-1} lambda_l cos(l theta), theta = -p in [0, pi]
-    // (entries l >= m hold 0), by Clenshaw's recurrence in FP64 (2 operations
-    // per term; gfx950 issues FP64 FMAs at the non-packed FP32 rate):
-    //     b_l = lambda_l + 2x b_{l+1} - b_{l+2},  sum_{l>=1} = x b_1 - b_2.
-    const double x = cos_theta_of(p);
-    if (cos_theta)
-        *cos_theta = x;
-    const double x2 = x + x;
-    double b1 = 0.0, b2 = 0.0;
-#pragma unroll
-    for (int l = M - 1; l >= 1; --l)
-    {
-        const double t = fma(x2, b1, (double)lam[l] - b2);
-        b2 = b1;
-        b1 = t;
-    }
-    return fma(2.0, fma(x, b1, -b2), (double)lam[0]);
-}
-
-// series_clenshaw at two phases in one pass, each recurrence with
-// series_clenshaw's operations, so both values are series_clenshaw's bit for
-// bit (the compiler runs the two recurrences one after the other; forced to
-// interleave them term by term, the march took as long)
-template <int M, typename L>
-__device__ __forceinline__ void series_clenshaw2(const L (&lam)[M], float pa, float pb, double &sa, double &sb)
-{
-    const double xa = cos_theta_of(pa), xb = cos_theta_of(pb);
-    const double x2a = xa + xa, x2b = xb + xb;
-    double a1 = 0.0, a2 = 0.0, b1 = 0.0, b2 = 0.0;
-#pragma unroll
-    for (int l = M - 1; l >= 1; --l)
-    {
-        const double ta = fma(x2a, a1, (double)lam[l] - a2);
-        const double tb = fma(x2b, b1, (double)lam[l] - b2);
-        a2 = a1;
-        a1 = ta;
-        b2 = b1;
-        b1 = tb;
-    }
-    sa = fma(2.0, fma(xa, a1, -a2), (double)lam[0]);
-    sb = fma(2.0, fma(xb, b1, -b2), (double)lam[0]);
+    cheb_low<block_width<M>()>(T, cos_theta_of(p));
+    return block_series<M>(c, T);
 }
 
 // fast_atan with the reciprocal from the hardware approximation (about one
@@ -261,6 +229,8 @@ __device__ __forceinline__ float fast_atan_rcp(float tan)
     x = __builtin_fmaf(x, y, z);
     return negative ? (-x) : x;
 }
+
+template <int M> constexpr bool kTwoSteps = M <= 96;
 
 // LagT: float multipliers, or FP64 ones kept from mray_hip_prepare_f64
 template <int M, typename LagT = float>
@@ -306,8 +276,9 @@ __global__ __launch_bounds__(256) void reconstruct_mixed_kernel(DevCamera cam, R
     for (int l = 0; l < M; ++l)
     {
         const LagT v = lag[off + min(l, nm - 1)];
-        lam[l] = (l < nm) ? (double)v : 0.0;
+        lam[l] = (l < nm) ? (l ? 2.0 : 1.0) * (double)v : 0.0;
     }
+    block_coefficients<M>(lam);
     float blo = 0.f, bhi = 1.f;
     if (bounds)
     {
@@ -322,15 +293,9 @@ __global__ __launch_bounds__(256) void reconstruct_mixed_kernel(DevCamera cam, R
         const float rho = fourier ? s : __builtin_fmaf(fast_atan_rcp(s), 0.318309886f, 0.5f);
         return __builtin_fmaf(rho, brange, blo);
     };
-    auto recon = [&](float p) { return density_of(series_clenshaw<M>(lam, rclamp(p, (float)(-kPi), 0.0f))); };
-    // the densities at p + dphi and p + 2 dphi (the march's float phase
-    // steps), from one interleaved pass
-    auto recon2 = [&](float p, float dphi, float &d1, float &d2) {
-        const float p1 = p + dphi, p2 = p1 + dphi;
-        double s1, s2;
-        series_clenshaw2<M>(lam, rclamp(p1, (float)(-kPi), 0.0f), rclamp(p2, (float)(-kPi), 0.0f), s1, s2);
-        d1 = density_of(s1);
-        d2 = density_of(s2);
+    auto recon = [&](float p) {
+        double T[block_width<M>() + 1];
+        return density_of(series_at<M>(lam, rclamp(p, (float)(-kPi), 0.0f), T));
     };
 
     Ray r = pixel_ray(cam, a.W, a.H, x, y);
@@ -366,17 +331,15 @@ __global__ __launch_bounds__(256) void reconstruct_mixed_kernel(DevCamera cam, R
             return stop;
         };
         // the loop (t <= t_far, at most cap steps, early termination) two
-        // steps at a time: both back samples from one pass (the second unused
-        // when the first step ends the march), half the loop's tests and
-        // branches; above 96 moments one at a time (the second sample's
-        // registers would cost occupancy)
+        // steps at a time: both back samples together (the second unused when
+        // the first step ends the march), half the loop's tests and branches
         int it = 0;
-        if constexpr (M <= 96)
+        if constexpr (kTwoSteps<M>)
         {
             while (t <= t_far && it < cap)
             {
-                float b1, b2;
-                recon2(p, dphi, b1, b2);
+                const float p1 = p + dphi;
+                const float b1 = recon(p1), b2 = recon(p1 + dphi);
                 if (step(b1))
                     break;
                 ++it;
@@ -623,7 +586,7 @@ __device__ __forceinline__ float fast_atan_deriv(float t)
 // entries from fs and its weight from frac(256 bs), so only bs carries a
 // derivative: d c / d bs = 256 (T[x1] - T[x0]). Then
 // d rho / d S = fast_atan'(S) / pi (hi - lo) and dS / d lambda_l = c_l cos(l theta)
-// (c_0 = 1, c_l = 2), cos(l theta) by the Chebyshev recurrence in FP64.
+// (c_0 = 1, c_l = 2): FP64 sums of products (block_sums), rounded to float once.
 // Transfer-function gradients are summed per workgroup in LDS and added to
 // grad_tf with one atomic per entry and workgroup. The LDS sums are 64-bit
 // fixed point (integer atomics: float atomics on LDS cost several times as
@@ -637,7 +600,7 @@ __device__ __forceinline__ float fast_atan_deriv(float t)
 // the shared series value, accumulates the gradient of its own multipliers,
 // and only lane 0 adds to the table gradient.
 template <int M, int K = 1>
-__global__ __launch_bounds__(256) void reconstruct_adjoint_kernel(
+__global__ __launch_bounds__(256, 2) void reconstruct_adjoint_kernel(
     DevCamera cam, RecArgs a, const float *__restrict__ lag, const uint32_t *__restrict__ index,
     const uint32_t *__restrict__ bounds, const float4 *__restrict__ tf_g, const float4 *__restrict__ rgba_fwd,
     const float4 *__restrict__ grad_rgba, float *__restrict__ grad_lag, float *__restrict__ grad_tf)
@@ -733,22 +696,32 @@ __global__ __launch_bounds__(256) void reconstruct_adjoint_kernel(
         }
         else
         {
-            float lam[M], glam[M];
+            // K = 1: the products' coefficients, and up to 40 moments (two
+            // wavefronts per SIMD) the products' sums, in FP64; else the lane's
+            // chunk of multipliers and of their gradient
+            constexpr bool kProducts = K == 1 && M <= 40;
+            using LamT = typename std::conditional<K == 1, double, float>::type;
+            using GradT = typename std::conditional<kProducts, double, float>::type;
+            LamT lam[M];
+            GradT glam[M];
 #pragma unroll
             for (int l = 0; l < M; ++l)
             {
                 const float v = lag[off + min(j0 + l, nm - 1)]; // unconditional, as in the forward
-                lam[l] = (j0 + l < nm) ? v : 0.0f;
-                glam[l] = 0.0f;
+                lam[l] = (j0 + l < nm) ? (LamT)v * (LamT)((K == 1 && l > 0) ? 2 : 1) : (LamT)0;
+                glam[l] = (GradT)0;
             }
-            // the series at phase pc; c1 = cos(theta), tj0 / tj0m1 = T_j0, T_j0-1
-            // of this lane's chunk (1 and cos(theta) for K = 1)
-            auto series_at = [&](float pc, double &c1, double &tj0, double &tj0m1) {
+            if constexpr (K == 1)
+                block_coefficients<M>(lam);
+            // the series at phase pc, with K = 1 leaving T_r of its cos(theta);
+            // else c1 = cos(theta), tj0 / tj0m1 = T_j0, T_j0-1 of this lane's chunk
+            double cheb[block_width<M>() + 1];
+            auto series = [&](float pc, double &c1, double &tj0, double &tj0m1) {
                 if constexpr (K == 1)
                 {
-                    const double sv = series_clenshaw<M>(lam, pc, &c1);
+                    const double sv = series_at<M>(lam, pc, cheb);
+                    c1 = tj0m1 = cheb[1];
                     tj0 = 1.0;
-                    tj0m1 = c1;
                     return sv;
                 }
                 else
@@ -777,7 +750,7 @@ __global__ __launch_bounds__(256) void reconstruct_adjoint_kernel(
                     return __builtin_fmaf(rho, brange, blo);
                 };
                 double c1, tj0, tj0m1;
-                float fs = rho_of((float)series_at(rclamp(p, (float)(-kPi), 0.0f), c1, tj0, tj0m1));
+                float fs = rho_of((float)series(rclamp(p, (float)(-kPi), 0.0f), c1, tj0, tj0m1));
                 double pre[3] = {0.0, 0.0, 0.0};
                 // table gradient of the current entry pair (x0, x1), not yet in gtf
                 int tf_x0 = -1, tf_x1 = -1;
@@ -798,7 +771,7 @@ __global__ __launch_bounds__(256) void reconstruct_adjoint_kernel(
                     t += a.step;
                     p += dphi;
                     const float pc = rclamp(p, (float)(-kPi), 0.0f);
-                    const float S = (float)series_at(pc, c1, tj0, tj0m1);
+                    const float S = (float)series(pc, c1, tj0, tj0m1);
                     const float bs = rho_of(S);
                     const float4 c = tf_sample_mixed(tf, fs, bs);
 
@@ -843,17 +816,22 @@ __global__ __launch_bounds__(256) void reconstruct_adjoint_kernel(
                     const float dS = (float)drho * brange * (fourier ? 1.0f : fast_atan_deriv(S) * 0.318309886f);
                     if (dS != 0.0f)
                     {
-                        // cos(l theta), theta = -pc, by the Chebyshev recurrence
-                        // from the series' own cos(theta), over the lane's
-                        // chunk l = j0 .. j0 + M - 1
-                        double cm = tj0m1, cl = tj0;
-#pragma unroll
-                        for (int l = 0; l < M; ++l)
+                        // dS cos(l theta), theta = -pc, on the series' own
+                        // cos(theta): the products' sums, or by the Chebyshev
+                        // recurrence over the lane's chunk l = j0 .. j0 + M - 1
+                        if constexpr (kProducts)
+                            block_sums<M, 0>(glam, (double)dS, cheb);
+                        else
                         {
-                            glam[l] = __builtin_fmaf(dS, (float)cl, glam[l]);
-                            const double cn = fma(2.0 * c1, cl, -cm);
-                            cm = cl;
-                            cl = cn;
+                            double cm = tj0m1, cl = tj0;
+#pragma unroll
+                            for (int l = 0; l < M; ++l)
+                            {
+                                glam[l] = __builtin_fmaf(dS, (float)cl, glam[l]);
+                                const double cn = fma(2.0 * c1, cl, -cm);
+                                cm = cl;
+                                cl = cn;
+                            }
                         }
                     }
                     tau += c.w;
@@ -867,11 +845,13 @@ __global__ __launch_bounds__(256) void reconstruct_adjoint_kernel(
             }
             if (grad_lag)
             {
+                if constexpr (kProducts)
+                    untangle_sums<M>(glam);
                 // static indices keep glam in registers
 #pragma unroll
                 for (int l = 0; l < M; ++l)
                     if (j0 + l < nm)
-                        grad_lag[off + j0 + l] = (j0 + l == 0) ? glam[l] : 2.0f * glam[l];
+                        grad_lag[off + j0 + l] = (float)((j0 + l == 0) ? glam[l] : (GradT)2 * glam[l]);
             }
         }
     }
