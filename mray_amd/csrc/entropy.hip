@@ -49,6 +49,7 @@ constexpr double kLsb = 1.0 / 16777216.0 / 16777216.0;    // AC__LeastSignifBit
 constexpr double kLeak = 2.0 * kLsb;                      // AC__Leakage
 constexpr uint32_t kMaxCount = 1u << 17;                  // DM__MaxCount
 constexpr int kMaxBits = 14;                              // 2^14 symbols at most
+constexpr int kLaneBits = 11;                             // alphabets decoded by LaneDecoder
 
 struct EntropyTable
 {
@@ -233,6 +234,21 @@ __device__ __forceinline__ uint64_t lanes_below()
     return (lane == 0) ? 0ull : (~0ull >> (64 - lane));
 }
 
+// the number of the last of the lanes (of a mask) for which p holds, p holding
+// for a prefix of them (0 if for none); the same in all lanes, by scalar
+// operations
+__device__ __forceinline__ int last_of_prefix(bool p, uint64_t lanes = ~0ull)
+{
+    return (int)__popcll((__ballot(p) & lanes) | 1ull) - 1;
+}
+
+// whether a carry or a renormalisation may be due (base >= 1 or length <=
+// 2^-16, or length next above it), by the doubles' high words
+__device__ __forceinline__ bool may_move(double base, double length)
+{
+    return (uint32_t)__double2hiint(base) >= 0x3FF00000u || __double2hiint(length) <= 0x3EF00000;
+}
+
 // the first k set bits of mask
 __device__ __forceinline__ uint64_t first_bits(uint64_t mask, uint32_t k)
 {
@@ -248,66 +264,104 @@ __device__ __forceinline__ uint64_t first_bits(uint64_t mask, uint32_t k)
     return out;
 }
 
-// The encoder's state (Arithmetic_Codec in mode 1): interval, and the code
-// bytes written by lane 0 into out[0, cap).
+// The encoder's state (Arithmetic_Codec in mode 1): the interval, and the code
+// as 16-bit digits (a renormalisation shifts out two bytes). The newest digits
+// are in an LDS ring of 128; a carry adds 1 to the newest one without looking
+// at it, and the digits are brought into [0, 2^16) when 64 of them leave the
+// ring together (flush). The newest digit always stays, so that a carry finds
+// its digit in the ring.
 struct Encoder
 {
     double base, length;
     uint8_t *out;
-    size_t pos, cap;
-    bool overflow;
+    size_t cap;
+    uint32_t *ring;        // 128 digits in LDS
+    uint32_t nd, flushed;  // digits so far, and of them in out
 
-    __device__ __forceinline__ void put(uint32_t b)
+    __device__ __forceinline__ void put(uint32_t a)
     {
         if (threadIdx.x == 0)
-        {
-            if (pos < cap)
-                out[pos] = (uint8_t)b;
-            else
-                overflow = true;
-        }
-        ++pos;
+            ring[nd & 127u] = a;
+        ++nd;
+        if (nd - flushed >= 96u)
+            flush(64u);
     }
 
     // propagate_carry (src/entropy_coding/arithmetic_codec.cpp:76-84)
     __device__ __forceinline__ void carry()
     {
         base -= 1.0;
-        if (threadIdx.x == 0)
+        if (threadIdx.x == 0 && nd > 0)
+            atomicAdd(&ring[(nd - 1u) & 127u], 1u);
+    }
+
+    // the next n <= 64 digits of the ring to out
+    __device__ __forceinline__ void flush(uint32_t n)
+    {
+        __syncthreads();
+        const uint32_t lane = threadIdx.x;
+        uint32_t v = (lane < n) ? ring[(flushed + lane) & 127u] : 0u;
+        uint32_t carried = 0;
+        while (__ballot(v > 0xFFFFu))
         {
-            size_t p = pos - 1;
-            while (p < cap && out[p] == 0xFFu)
-                out[p--] = 0;
-            if (p < cap)
-                out[p] = (uint8_t)(out[p] + 1);
+            const uint32_t c = v >> 16;
+            carried += (uint32_t)__builtin_amdgcn_readfirstlane((int)c);
+            const uint32_t up = __shfl_down(c, 1);
+            v = (v & 0xFFFFu) + (lane < 63u ? up : 0u);
         }
+        const size_t at = 2 * (size_t)(flushed + lane);
+        if (carried)
+        {
+            // into the bytes already out
+            __threadfence();
+            if (lane == 0)
+            {
+                size_t p = 2 * (size_t)flushed - 1;
+                while (p < cap && out[p] == 0xFFu)
+                    out[p--] = 0;
+                if (p < cap)
+                    out[p] = (uint8_t)(out[p] + 1);
+            }
+            __threadfence();
+        }
+        if (lane < n)
+        {
+            if (at < cap)
+                out[at] = (uint8_t)(v >> 8);
+            if (at + 1 < cap)
+                out[at + 1] = (uint8_t)v;
+        }
+        flushed += n;
+        __syncthreads();
     }
 
     // encode(data, Adaptive_Data_Model) with the symbol's d(s) and d(s + 1)
-    // (:445-475), the model update done by the caller
-    __device__ __forceinline__ void encode(double lo, double hi, bool last)
+    // (1 for the last symbol) (:445-475), the model update done by the caller
+    __device__ __forceinline__ void encode(double lo, double hi)
     {
-        const double y = last ? base + length : base + length * hi;
+        const double y = base + length * hi;
         base += length * lo;
         length = y - base;
-        if (base >= 1.0)
-            carry();
-        if ((length -= kLeak) <= kMinLength)
+        length -= kLeak;
+        // one rarely taken branch for both: about every third symbol
+        if (may_move(base, length))
         {
+            if (base >= 1.0)
+                carry();
             // renorm_enc_interval (:87-97)
-            do
+            while (length <= kMinLength)
             {
                 base *= kOut;
                 const uint32_t a = (uint32_t)base;
-                put(a >> 8);
-                put(a & 0xFFu);
+                put(a);
                 base -= (double)a;
-            } while ((length *= kOut) <= kMinLength);
+                length *= kOut;
+            }
         }
     }
 
-    // stop_encoder (:631-675)
-    __device__ void finish()
+    // stop_encoder (:631-675); the code's size in bytes
+    __device__ size_t finish()
     {
         const uint32_t a = (uint32_t)(kOut * base), b = (uint32_t)(kOut * (base + length));
         int last;
@@ -328,13 +382,19 @@ struct Encoder
         }
         if (base >= 1.0)
             carry();
+        while (flushed < nd)
+            flush(min(64u, nd - flushed));
+        size_t pos = 2 * (size_t)nd;
         do
         {
             base *= 256.0;
             const uint32_t c = (uint32_t)base;
-            put(c);
+            if (threadIdx.x == 0 && pos < cap)
+                out[pos] = (uint8_t)c;
+            ++pos;
             base -= (double)c;
         } while (--last);
+        return pos;
     }
 };
 
@@ -348,7 +408,7 @@ __global__ __launch_bounds__(64) void entropy_encode_kernel(const float *__restr
                                                             uint16_t *__restrict__ zeroth,
                                                             uint64_t *__restrict__ sizes)
 {
-    extern __shared__ uint32_t lds_model[];
+    extern __shared__ __align__(16) uint32_t lds_model[];
     const int l = blockIdx.x;
     const int lane = threadIdx.x;
     float lo, hi;
@@ -376,7 +436,8 @@ __global__ __launch_bounds__(64) void entropy_encode_kernel(const float *__restr
 
     Model M;
     M.reset(lds_model, 1u << bits);
-    Encoder E{0.0, 1.0, streams + stream_off[l - 1], 0, (size_t)(stream_off[l] - stream_off[l - 1]), false};
+    __shared__ uint32_t ring[128];
+    Encoder E{0.0, 1.0, streams + stream_off[l - 1], (size_t)(stream_off[l] - stream_off[l - 1]), ring, 0u, 0u};
     for (uint32_t p0 = 0; p0 < npix; p0 += 64)
     {
         const uint32_t p = p0 + lane;
@@ -397,15 +458,14 @@ __global__ __launch_bounds__(64) void entropy_encode_kernel(const float *__restr
             if (mine)
             {
                 dlo = M.d(sym);
-                dhi = last ? 0.0 : M.d(sym + 1);
+                dhi = last ? 1.0 : M.d(sym + 1);
             }
-            const uint64_t lastmask = __ballot(mine && last);
             uint64_t s = seg;
             while (s)
             {
                 const int i = __ffsll((unsigned long long)s) - 1;
                 s &= s - 1;
-                E.encode(readlane_f64(dlo, i), readlane_f64(dhi, i), (lastmask >> i) & 1ull);
+                E.encode(readlane_f64(dlo, i), readlane_f64(dhi, i));
             }
             if (mine)
                 atomicAdd(&M.count[sym], 1u);
@@ -415,9 +475,9 @@ __global__ __launch_bounds__(64) void entropy_encode_kernel(const float *__restr
                 M.update();
         }
     }
-    E.finish();
+    const size_t size = E.finish();
     if (lane == 0)
-        sizes[l] = E.overflow ? ~0ull : (uint64_t)E.pos;
+        sizes[l] = size > E.cap ? ~0ull : (uint64_t)size;
 }
 
 // The decoder's state (Arithmetic_Codec in mode 2); bytes past the code's
@@ -541,13 +601,255 @@ struct Decoder
     }
 };
 
+// The model with its distribution in registers, for alphabets of up to 2^8
+// symbols (R = 1, 2, 4 symbols per lane): lane i holds d(iR) .. d(iR + R),
+// infinity from the alphabet's end on (such a symbol never qualifies), d(A) as
+// 1 (base + length * 1 is the reference's base + length).
+// Above (R = 0, up to 2^11 symbols) the lanes hold the 64 block starts and the
+// block's at most 32 ends are read from LDS (dist).
+template <int R> struct LaneModel
+{
+    uint32_t *count; // LDS
+    double *dist;    // LDS, A + 1 entries (R = 0)
+    uint32_t A, total, cycle, until;
+    uint32_t shift; // log2 (A / 64) (R = 0)
+    double d[R + 1];
+
+    __device__ __forceinline__ uint32_t per() const { return R ? (uint32_t)R : A / 64u; }
+
+    // update() (see Model)
+    __device__ __forceinline__ void update()
+    {
+        const uint32_t lane = threadIdx.x, n = per(), k0 = lane * n;
+        __syncthreads();
+        total += cycle;
+        const bool halve = total > kMaxCount;
+        uint32_t part = 0;
+        for (uint32_t r = 0; r < n; ++r)
+            if (k0 + r < A)
+            {
+                uint32_t c = count[k0 + r];
+                if (halve)
+                    count[k0 + r] = c = (c + 1) >> 1;
+                part += c;
+            }
+        if (halve)
+            total = wave_sum_u32(part);
+        uint32_t run = wave_exclusive_scan_u32(part);
+        const double scale = 1.0 / (double)total;
+        if constexpr (R > 0)
+        {
+#pragma unroll
+            for (int r = 0; r <= R; ++r)
+            {
+                const uint32_t k = k0 + (uint32_t)r;
+                d[r] = (k < A) ? scale * (double)run : (r == R && k == A) ? 1.0 : __builtin_inf();
+                if (r < R && k < A)
+                    run += count[k];
+            }
+        }
+        else
+        {
+            d[0] = scale * (double)run;
+            for (uint32_t r = 0; r < n; ++r)
+            {
+                dist[k0 + r] = scale * (double)run;
+                run += count[k0 + r];
+            }
+            if (lane == 0)
+                dist[A] = 1.0;
+        }
+        cycle = (5 * cycle) >> 2;
+        const uint32_t cap = (A + 6) << 3;
+        if (cycle > cap)
+            cycle = cap;
+        until = cycle;
+        __syncthreads();
+    }
+
+    __device__ void reset(uint32_t *lds, uint32_t alphabet)
+    {
+        A = alphabet;
+        dist = reinterpret_cast<double *>(lds);
+        shift = R ? 0u : 25u - (uint32_t)__clz((int)A);
+        count = lds + (R ? 0u : 2u * (A + 2u));
+        for (uint32_t k = threadIdx.x; k < A; k += 64)
+            count[k] = 1;
+        total = 0;
+        cycle = A;
+        update();
+        cycle = until = (A + 6) >> 1;
+    }
+};
+
+// The decoder on a LaneModel: no table, and LDS only for the second level of
+// large alphabets. All candidates' ends are formed at once; they increase
+// strictly with k, so the number of lanes whose first end is at or below the
+// value names the lane, which has already chosen among its R symbols. The next
+// two code bytes wait as value increment; lane i holds digit wat + i of the
+// code and of the 64 after it.
+struct LaneDecoder
+{
+    double base, length, value, next;
+    const uint8_t *in;
+    size_t n;
+    size_t loaded;       // digits loaded so far (128 ahead at most)
+    uint32_t win, ahead; // 64 digits each
+    uint32_t at;         // next digit in win
+
+    __device__ __forceinline__ uint32_t load(size_t digit) const
+    {
+        const size_t q = 6 + 2 * (digit + threadIdx.x);
+        const uint32_t b0 = q < n ? in[q] : 0u, b1 = q + 1 < n ? in[q + 1] : 0u;
+        return b0 << 8 | b1;
+    }
+
+    // the next digit's value increment, kLsb (256 b0 + b1) (exact)
+    __device__ __forceinline__ void fetch()
+    {
+        if (at == 64u)
+        {
+            win = ahead;
+            ahead = load(loaded);
+            loaded += 64;
+            at = 0;
+        }
+        next = kLsb * (double)(uint32_t)__builtin_amdgcn_readlane((int)win, (int)at);
+        ++at;
+    }
+
+    // start_decoder (:590-604)
+    __device__ void start(const uint8_t *code, size_t size)
+    {
+        in = code;
+        n = size;
+        length = 1.0;
+        base = value = 0.0;
+        for (size_t k = 0; k < 6; ++k)
+            value = 256.0 * value + kLsb * (double)(k < n ? in[k] : 0u);
+        win = load(0);
+        ahead = load(64);
+        loaded = 128;
+        at = 0;
+        fetch();
+    }
+
+    // decode(Adaptive_Data_Model) (:477-519) without the model's count update
+    template <int R> __device__ __forceinline__ uint32_t decode(const LaneModel<R> &M)
+    {
+        const double sv = value + kLsb;
+        uint32_t s;
+        double x, y;
+        if constexpr (R > 0)
+        {
+            double z[R + 1];
+#pragma unroll
+            for (int r = 0; r <= R; ++r)
+                z[r] = base + length * M.d[r];
+            // with none qualifying symbol 0, as the reference's bisection
+            const int j = last_of_prefix(!(z[0] > sv));
+            double xl = z[0], yl = z[1];
+            uint32_t sub = 0;
+#pragma unroll
+            for (int r = 1; r < R; ++r)
+            {
+                const bool q = !(z[r] > sv);
+                xl = q ? z[r] : xl;
+                yl = q ? z[r + 1 <= R ? r + 1 : R] : yl;
+                sub = q ? (uint32_t)r : sub;
+            }
+            x = readlane_f64(xl, j);
+            y = readlane_f64(yl, j);
+            s = (uint32_t)j * R;
+            if constexpr (R > 1)
+                s += (uint32_t)__builtin_amdgcn_readlane((int)sub, j);
+        }
+        else
+        {
+            const double zc = base + length * M.d[0];
+            const uint32_t n = M.A / 64u, i = min((uint32_t)threadIdx.x, n);
+            const uint32_t k0 = (uint32_t)last_of_prefix(!(zc > sv)) << M.shift;
+            const double z = base + length * M.dist[k0 + i];
+            const int j = last_of_prefix(!(z > sv), (1ull << n) - 1ull);
+            x = readlane_f64(z, j);
+            y = readlane_f64(z, j + 1);
+            s = k0 + (uint32_t)j;
+        }
+        base = x;
+        length = y - x;
+        length -= kLeak;
+        if (may_move(base, length))
+        {
+            if (base >= 1.0)
+            {
+                base -= 1.0;
+                value -= 1.0;
+            }
+            // renorm_dec_interval (:101-112)
+            while (length <= kMinLength)
+            {
+                base *= kOut;
+                const double a = (double)(uint32_t)base;
+                base -= a;
+                value = (kOut * value - a) + next;
+                length *= kOut;
+                fetch();
+            }
+        }
+        return s;
+    }
+};
+
+template <int R>
+__device__ void decode_stream(uint32_t *lds, uint32_t alphabet, const uint8_t *code, size_t size,
+                              const uint32_t *__restrict__ index, uint32_t npix, uint32_t l, int bits, float lo,
+                              float hi, float *__restrict__ data)
+{
+    const int lane = threadIdx.x;
+    LaneModel<R> M;
+    M.reset(lds, alphabet);
+    LaneDecoder D;
+    D.start(code, size);
+    for (uint32_t p0 = 0; p0 < npix; p0 += 64)
+    {
+        const uint32_t p = p0 + lane;
+        uint32_t start = 0, n = 0;
+        if (p < npix)
+            n = count_of(index, p, start);
+        const bool has = n > l;
+        uint64_t mask = __ballot(has);
+        uint32_t mine = 0;
+        while (mask)
+        {
+            // the symbols up to the next model update share one model
+            const uint64_t seg = first_bits(mask, M.until);
+            uint64_t todo = seg;
+            while (todo)
+            {
+                const int i = __ffsll((unsigned long long)todo) - 1;
+                todo &= todo - 1;
+                const uint32_t s = D.decode(M);
+                mine = (lane == i) ? s : mine;
+            }
+            if ((seg >> lane) & 1ull)
+                atomicAdd(&M.count[mine], 1u);
+            M.until -= (uint32_t)__popcll(seg);
+            mask &= ~seg;
+            if (M.until == 0)
+                M.update();
+        }
+        if (has)
+            data[start + l] = ent_dequantize(mine, bits, lo, hi);
+    }
+}
+
 __global__ __launch_bounds__(64) void entropy_decode_kernel(const uint8_t *__restrict__ section,
                                                             const uint64_t *__restrict__ code_off,
                                                             const uint32_t *__restrict__ index, uint32_t npix,
                                                             int prediction_coded, EntropyTable t,
                                                             float *__restrict__ data)
 {
-    extern __shared__ uint32_t lds_model[];
+    extern __shared__ __align__(16) uint32_t lds_model[];
     const int l = blockIdx.x;
     const int lane = threadIdx.x;
     float lo, hi;
@@ -578,13 +880,29 @@ __global__ __launch_bounds__(64) void entropy_decode_kernel(const uint8_t *__res
         return;
     }
 
+    const uint8_t *code = section + code_off[2 * l];
+    const size_t code_size = (size_t)(code_off[2 * l + 1] - code_off[2 * l]);
+    if (bits <= kLaneBits)
+    {
+        const uint32_t A = 1u << bits, ul = (uint32_t)l;
+        if (bits <= 6)
+            decode_stream<1>(lds_model, A, code, code_size, index, npix, ul, bits, lo, hi, data);
+        else if (bits == 7)
+            decode_stream<2>(lds_model, A, code, code_size, index, npix, ul, bits, lo, hi, data);
+        else if (bits == 8)
+            decode_stream<4>(lds_model, A, code, code_size, index, npix, ul, bits, lo, hi, data);
+        else
+            decode_stream<0>(lds_model, A, code, code_size, index, npix, ul, bits, lo, hi, data);
+        return;
+    }
+
     Model M;
     M.reset(lds_model, 1u << bits);
     uint16_t *tab = reinterpret_cast<uint16_t *>(lds_model + 2 * M.A);
     build_table(M, tab);
     // stream l: [code_off[2 l], code_off[2 l + 1])
     Decoder D;
-    D.start(section + code_off[2 * l], (size_t)(code_off[2 * l + 1] - code_off[2 * l]));
+    D.start(code, code_size);
     for (uint32_t p0 = 0; p0 < npix; p0 += 64)
     {
         const uint32_t p = p0 + lane;
@@ -815,7 +1133,11 @@ int launch_entropy_decode(const uint8_t *in, size_t n_in, const uint32_t *index,
     if (hipMallocAsync((void **)&buf, sec_b + off.size() * sizeof(uint64_t), stream) != hipSuccess)
         return MRAY_ERR_OOM;
     uint64_t *d_off = reinterpret_cast<uint64_t *>(buf + sec_b);
-    const size_t lds = (size_t)amax * 2 * sizeof(uint32_t) + kTabEntries * sizeof(uint16_t);
+    // up to kLaneBits the counts and an FP64 distribution of A + 1 entries
+    // (padded to A + 2), above the counts, running sums and lookup table
+    const size_t lds = (amax <= (1u << kLaneBits))
+                           ? (size_t)amax * sizeof(uint32_t) + ((size_t)amax + 2) * sizeof(double)
+                           : (size_t)amax * 2 * sizeof(uint32_t) + kTabEntries * sizeof(uint16_t);
     rc = set_lds(reinterpret_cast<const void *>(entropy_decode_kernel), lds);
     if (rc == 0 && (hipMemcpyAsync(buf, in, (size_t)pos, hipMemcpyHostToDevice, stream) != hipSuccess ||
                     hipMemcpyAsync(d_off, off.data(), off.size() * sizeof(uint64_t), hipMemcpyHostToDevice, stream) !=
