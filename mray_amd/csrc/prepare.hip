@@ -55,19 +55,6 @@ __global__ __launch_bounds__(64) void prepare_plain_kernel(const float *__restri
 // MIXED (FP64, G lanes per pixel)
 // ---------------------------------------------------------------------------
 
-// 2 pi / j
-struct TwoPiOver
-{
-    double v[256];
-    constexpr TwoPiOver() : v()
-    {
-        v[0] = 0.0;
-        for (int j = 1; j < 256; ++j)
-            v[j] = 2.0 * kPi / j;
-    }
-};
-__constant__ TwoPiOver kTwoPiOver;
-
 // For the Hermitian Toeplitz matrix of t (t_0 real) the lattice of order n
 //     a^n = a^n-1 + k z b^n-1,        b^n = z b^n-1 + conj(k) a^n-1
 // gives the (monic) solution polynomial a and its reverse b; the sequences
@@ -119,106 +106,15 @@ __global__ __launch_bounds__(64, 2) void prepare_mixed_kernel(const float *__res
 
     dc *E = lds_c + q * S;
     double *T = reinterpret_cast<double *>(E);
-    // biased moments, lerp in FP64 (near the boundary of the moment space the
-    // recursion below amplifies a one-ulp change of the input); through LDS
-    // from the coalesced order of the loads to the lanes' blocks
-    const double b64 = (double)bias;
-#pragma unroll
-    for (int r = 0; r < C; ++r)
-    {
-        const int e = G * r + g;
-        const double v = (e < nm) ? (double)mom[off + e] : 0.0;
-        T[e] = (e < nm) ? (1.0 - b64) * v + (e == 0 ? b64 * 0.5 : 0.0) : 0.0;
-    }
-    T[N] = 0.0; // element N of the shifted weights (the stride holds 2 N + 2 doubles)
-    wave_sync();
     double V[C];
-#pragma unroll
-    for (int c = 0; c < C; ++c)
-        V[c] = (double)(g * C + c + 1) * T[g * C + c + 1];
-    const double t0 = (nm > 0) ? T[0] : 0.5;
-    wave_sync();
-
-    // Herglotz transform: trigonometric -> exponential moments
-    // (trigonometricToExponentialMoments, src/mese/MESE_dynamic.h:35-54)
+    const double t0 = load_weights<G, C>(mom, off, nm, (double)bias, g, T, V);
     double sn, cs;
     sincos(kPi * t0 - 0.5 * kPi, &sn, &cs);
     const dc e0 = dc{cs * (0.25 / kPi), sn * (0.25 / kPi)};
-    if (g == 0)
-        E[0] = (nm > 0) ? e0 : dc{0.0, 0.0};
-    {
-        dc X[C];
-#pragma unroll
-        for (int c = 0; c < C; ++c)
-            X[c] = dc{V[c] * e0.x, V[c] * e0.y};
-        for (int j = 1; j < nw; ++j)
-        {
-            const double f = kTwoPiOver.v[j];
-            const dc x0 = bcast0<G>(X[0]);
-            const dc ej = dc{-f * x0.y, f * x0.x};
-            if (g == 0)
-                E[j] = (j < nm) ? ej : dc{0.0, 0.0};
-            const dc nx = shl1<G>(X[0], last);
-#pragma unroll
-            for (int c = 0; c < C; ++c)
-            {
-                const dc xn = (c + 1 < C) ? X[c + 1 < C ? c + 1 : 0] : nx;
-                X[c] = dc{fma_moved(V[c], ej.x, xn.x), fma_moved(V[c], ej.y, xn.y)};
-            }
-        }
-    }
-    // the correlation reads E four at a time
-    static_assert(N % 4 == 0, "E is read up to the next multiple of four");
-    if (g < 4 && nw + g < N)
-        E[nw + g] = dc{0.0, 0.0};
-    wave_sync();
-
-    // the lattice (levinsonsAlgorithm, src/mese/MESE_dynamic.h:100-135)
-    dc F[C], B[C];
-#pragma unroll
-    for (int c = 0; c < C; ++c)
-    {
-        const int i = g * C + c;
-        const dc e = E[min(i, nw - 1)];
-        F[c] = (i < nw) ? e : dc{0.0, 0.0};
-        B[c] = (i < nw - 1) ? e : (i == nw - 1) ? dc{1.0, 0.0} : dc{0.0, 0.0};
-        if (c == 0 && g == 0 && nw > 1)
-            B[c] = dc{2.0 * e0.x, 0.0};
-    }
-    double rs = 1.0 / (2.0 * e0.x); // 1 / sigma
-    bool valid = true;
-    for (int L = (nw - 2) / C; L >= 0; --L)
-    {
-#pragma unroll
-        for (int cs = C - 1; cs >= 0; --cs)
-        {
-            const int seam = L * C + cs; // n = nw - 2 - seam steps are done
-            if (seam > nw - 2)
-                continue;
-            const dc f1 = bcast0<G>(F[1]);
-            dc k = dc{-f1.x * rs, -f1.y * rs};
-            double k2 = fma(k.x, k.x, k.y * k.y);
-            if (!valid || nw - 1 - seam >= nm || k2 >= 1.0)
-            {
-                k = dc{0.0, 0.0};
-                k2 = 0.0;
-                valid = false;
-            }
-            rs *= recip_nr(1.0 - k2);
-            const dc nx = shl1<G>(F[0], last);
-#pragma unroll
-            for (int c = 0; c < C; ++c)
-            {
-                const dc f = (c + 1 < C) ? F[c + 1 < C ? c + 1 : 0] : nx, b = B[c];
-                F[c] = dc{fma(k.x, b.x, fma(-k.y, b.y, f.x)), fma(k.x, b.y, fma(k.y, b.x, f.y))};
-                B[c] = dc{fma(k.x, f.x, fma(k.y, f.y, b.x)), fma(k.x, f.y, fma(-k.y, f.x, b.y))};
-            }
-            if (g == L)
-                B[cs] = dc{k.x, -k.y};
-        }
-    }
-    if (g == 0)
-        F[0] = dc{1.0, 0.0};
+    herglotz<G, C>(V, e0, nw, nm, g, last, E);
+    dc F[C];
+    double rs;
+    lattice<G, C>(E, e0, nw, nm, g, last, F, rs);
 
     // autocorrelation of a (computeAutocorrelation): R_i = sum_j a_j conj(a_j+i)
     dc R[C];

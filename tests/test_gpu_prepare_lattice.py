@@ -87,3 +87,68 @@ def test_outside_the_moment_space(O, W, H):
     lag = hip.prepare(torch.from_numpy(mo).cuda(), W, H, m, 1e-3, form="mixed64").cpu().numpy().reshape(-1, m)
     pick = rng.integers(0, W * H, 30)
     check(O, mo[pick], lag[pick], np.full(30, m), 1e-3, 1e-9)
+
+
+def fd_gradient(O, mo, gl, bias, eps=1e-6):
+    """Central differences of sum(gl * prepare(mo)) in the FP64 oracle."""
+    out = np.empty(len(mo))
+    for j in range(len(mo)):
+        v = []
+        for s in (eps, -eps):
+            x = mo.astype(np.float64).copy()
+            x[j] += s
+            v.append(float(gl.astype(np.float64) @ O.prepare_std_f64(len(mo), x, float(np.float32(bias)))))
+        out[j] = (v[0] - v[1]) / (2 * eps)
+    return out
+
+
+# 4, 8 and 16 lanes per pixel (up to 40, 80 and 255 moments), their block edges
+@pytest.mark.parametrize("m", [1, 2, 8, 9, 39, 40, 41, 63, 80, 81, 160, 161, 255])
+def test_adjoint_against_differences(O, m):
+    """dL/dmoments against differences of the FP64 oracle. At MESE bias 0.05 the
+    solution's condition number stays below ~1e3, so the differences (step
+    1e-6) are good to ~1e-8 of the gradient's norm; the kernel rounds to f32
+    once: 1e-5 leaves both a factor of 100."""
+    W, H, bias = 3, 7, 0.05
+    rng = np.random.default_rng(m)
+    mo = densities(rng, W * H, m)
+    gl = rng.normal(size=(W * H, m)).astype(np.float32)
+    gm = hip.prepare_backward(torch.from_numpy(mo).cuda(), W, H, m, bias, torch.from_numpy(gl).cuda())
+    gm = gm.cpu().numpy().reshape(-1, m).astype(np.float64)
+    for i in (0, 10, W * H - 1):
+        ref = fd_gradient(O, mo[i], gl[i], bias)
+        assert np.linalg.norm(gm[i] - ref) <= 1e-5 * np.linalg.norm(ref), (i, np.linalg.norm(gm[i] - ref) / np.linalg.norm(ref))
+
+
+def test_adjoint_past_the_guard(O):
+    """Where the guard fires (order 12 of 24) the later coefficients are constants."""
+    W, H, m, bias = 4, 4, 24, 0.05
+    rng = np.random.default_rng(9)
+    mo = densities(rng, W * H, m)
+    mo[:, 12] += 3.0
+    gl = rng.normal(size=(W * H, m)).astype(np.float32)
+    gm = hip.prepare_backward(torch.from_numpy(mo).cuda(), W, H, m, bias, torch.from_numpy(gl).cuda())
+    gm = gm.cpu().numpy().reshape(-1, m).astype(np.float64)
+    for i in range(4):
+        ref = fd_gradient(O, mo[i], gl[i], bias)
+        assert np.linalg.norm(gm[i] - ref) <= 1e-5 * np.linalg.norm(ref)
+
+
+def test_adjoint_compact_matches_dense(O):
+    """Ragged counts with empty pixels, every lane group: a pixel's gradient does
+    not depend on the image's largest count (up to FP64 rounding, then f32)."""
+    W, H, bias = 9, 8, 0.05
+    rng = np.random.default_rng(3)
+    nm = rng.integers(0, 41, W * H)
+    nm[:5] = (0, 1, 2, 40, 39)
+    mo = densities(rng, W * H, 40)
+    index = np.concatenate([[0], np.cumsum(nm)]).astype(np.int32)
+    data = np.concatenate([mo[i][:nm[i]] for i in range(W * H)])
+    gl = rng.normal(size=len(data)).astype(np.float32)
+    dev = [torch.from_numpy(a).cuda() for a in (data, gl, index)]
+    out = [hip.prepare_backward(dev[0], W, H, m, bias, dev[1], index=dev[2]).cpu().numpy().astype(np.float64)
+           for m in (40, 64, 120, 255)]
+    for i in np.flatnonzero(nm):
+        a = slice(index[i], index[i + 1])
+        for o in out[1:]:
+            assert np.linalg.norm(o[a] - out[0][a]) <= 1e-6 * np.linalg.norm(out[0][a])
