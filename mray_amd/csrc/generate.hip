@@ -430,10 +430,9 @@ struct WeightRing
 // J0C: a chunk start known at compile time (!GRID).
 //
 // Measured (1024^3 f32, 1024 x 1024 rays, 50 moments): 11.6 ms node by node,
-// 8.1 ms gridded, 207 instead of 341 VALU instructions per node, 84 % of the
-// issue slots; 2048 x 2048 x 1920 u8, 2048 x 2048 rays, 100 moments: 132 and
-// 77 ms (the bytes' divisions and the corner addresses are a third of that
-// gain). Bound by VALU issue, then by load latency at two wavefronts per SIMD.
+// 7.1 ms gridded (8.1 before the corners came in pairs); 2048 x 2048 x 1920
+// u8, 2048 x 2048 rays, 100 moments: 132 and 76 ms (the bytes' divisions and
+// the corner addresses are a third of that gain). Bound by VALU issue, then by load latency at two wavefronts per SIMD.
 __device__ __forceinline__ bool grid_resolves(int m, float dphi, float t_near, float t_far, float s)
 {
     return (float)(m - 1) * dphi <= 1.0f && t_far <= 8192.0f * s && t_near + s < t_far;

@@ -11,7 +11,7 @@
 // the IEEE quotient), map_density, the table lookup with its weight quirk
 // (tf_sample), float compositing without contraction and T = exp(-tau) in
 // double, so the RGBA is bit-identical to the CPU oracle's. The next
-// sample's eight loads are issued one step ahead (PendingSample).
+// sample's loads are issued one step ahead (PendingSample).
 #include <hip/hip_runtime.h>
 
 #include "device_common.hpp"
@@ -110,7 +110,7 @@ int launch_typed(const T *vox, int nx, int ny, int nz, const float *dmin, const 
     const VolumeView<T> v = make_volume_view(vox, nx, ny, nz, dmin, dmax);
     const uint32_t ntiles = (uint32_t)(((a.W + 7) / 8) * ((a.H + 7) / 8));
     const dim3 grid((ntiles + 3) / 4);
-    // byte offsets of every voxel fit in 32 bits up to 4 GiB of volume
+    // pairs of voxels at 32-bit byte offsets, up to 4 GiB of volume
     const bool off32 = offsets_fit(nx, ny, nz, sizeof(T));
     if (off32)
         hipLaunchKernelGGL((reference_kernel<T, true>), grid, dim3(256), 0, stream, v, c, a, tf, rgba, steps);
