@@ -390,6 +390,19 @@ struct WeightRing
     }
 };
 
+// a value of another lane of the quad (CTRL: quad_perm)
+template <int CTRL> __device__ __forceinline__ float dpp_quad(float v)
+{
+    return __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), CTRL, 0xF, 0xF, true));
+}
+template <int CTRL> __device__ __forceinline__ double dpp_quad(double v)
+{
+    int2 w = __builtin_bit_cast(int2, v);
+    w.x = __builtin_amdgcn_update_dpp(0, w.x, CTRL, 0xF, 0xF, true);
+    w.y = __builtin_amdgcn_update_dpp(0, w.y, CTRL, 0xF, 0xF, true);
+    return __builtin_bit_cast(double, w);
+}
+
 // The integral per node. A segment [u, p] of the reference with slope g
 // contributes, with c(phi) = cos(j phi) and rho the line's values at its ends,
 //     (1/j^2) [ g c(p) - rho_p c'(p) - g c(u) + rho_u c'(u) ].
@@ -428,6 +441,12 @@ struct WeightRing
 // the sample counts); the CHUNK kernel runs the later ones,
 // j0 = (blockIdx.y + 1) M.
 // J0C: a chunk start known at compile time (!GRID).
+// S = 4: four lanes per ray, each the terms of a quarter of its nodes (from the
+// segment that ends at the first of them to the one that starts at the last),
+// their sums added at the end. For images of few rays, which leave most SIMDs
+// without a wavefront: a lone wavefront takes 0.5 us per node.
+// Measured (128^3, 30 moments): 100 steps, up to 16384 rays 62 us by one lane,
+// 28 by four; 1000 steps 541 and 179 (each lane first adds up its t).
 //
 // Measured (1024^3 f32, 1024 x 1024 rays, 50 moments): 11.6 ms node by node,
 // 7.1 ms gridded (8.1 before the corners came in pairs); 2048 x 2048 x 1920
@@ -438,7 +457,7 @@ __device__ __forceinline__ bool grid_resolves(int m, float dphi, float t_near, f
     return (float)(m - 1) * dphi <= 1.0f && t_far <= 8192.0f * s && t_near + s < t_far;
 }
 
-template <typename T, int M, bool OFF32, bool POW2, bool CHUNK, bool GRID, int J0C>
+template <typename T, int M, bool OFF32, bool POW2, bool CHUNK, bool GRID, int J0C, int S = 1>
 __global__ __launch_bounds__(256, 2) void generate_mixed_kernel(VolumeView<T> vol, DevCamera cam, GenArgs a,
                                                              float *__restrict__ out, uint32_t *__restrict__ bounds,
                                                              int32_t *__restrict__ samples,
@@ -447,12 +466,14 @@ __global__ __launch_bounds__(256, 2) void generate_mixed_kernel(VolumeView<T> vo
     const int tid = threadIdx.x;
     const int lane = tid & 63;
     const uint32_t ntiles = ((a.W + 7) / 8) * ((a.H + 7) / 8);
-    const uint32_t tile = xcd_tile_block(a.W, 4) * 4 + (tid >> 6);
+    static_assert(S == 1 || (S == 4 && GRID && !CHUNK), "four lanes per ray: the gridded march, unchunked");
+    const int quad = tid & 3; // S = 4: a workgroup's tile, 16 rays per wavefront
+    const uint32_t tile = S == 4 ? xcd_tile_block(a.W, 1) : xcd_tile_block(a.W, 4) * 4 + (tid >> 6);
     if (tile >= ntiles)
         return;
     int x, y;
-    tile_pixel(tile, a.W, lane, x, y);
-    if (x >= a.W || y >= a.H)
+    tile_pixel(tile, a.W, S == 4 ? tid >> 2 : lane, x, y);
+    if (S == 1 && (x >= a.W || y >= a.H))
         return;
     const int m = a.m;
     const int j0 = CHUNK ? (J0C ? J0C : (int)(blockIdx.y + 1) * M) : 0;
@@ -462,6 +483,17 @@ __global__ __launch_bounds__(256, 2) void generate_mixed_kernel(VolumeView<T> vo
     float t_near, t_far;
     bool hit = intersect_aabb(r, vol.dmin, vol.dmax, t_near, t_far);
     t_near = rmax(t_near, cam.znear);
+    bool tile_gridded = false;
+    if constexpr (S == 4)
+    {
+        // whether the tile's rays are gridded: as its wavefront decides in the
+        // other launch
+        const bool inside = x < a.W && y < a.H;
+        const float step_phase = (float)(kPi * (double)(a.step / (t_far - t_near)));
+        tile_gridded = !__syncthreads_or(inside && hit && t_far > 0 && !grid_resolves(m, step_phase, t_near, t_far, a.step));
+        if (!inside)
+            return;
+    }
     size_t pix = (size_t)y * a.W + x;
     float *mo = out + pix * (size_t)m;
     if (!(hit && (t_far > 0)))
@@ -487,7 +519,7 @@ __global__ __launch_bounds__(256, 2) void generate_mixed_kernel(VolumeView<T> vo
     const float pi_trange_inv = (float)(kPi / (double)(t_far - t_near));
     const float dphi = (float)(kPi * (double)(s / (t_far - t_near)));
     // by wavefront: whether its rays are gridded
-    const bool gridded = !__any(!grid_resolves(m, dphi, t_near, t_far, s));
+    const bool gridded = S == 4 ? tile_gridded : !__any(!grid_resolves(m, dphi, t_near, t_far, s));
     if (GRID ? !gridded : (gridded && a.rays == kRaysUngridded))
         return;
 
@@ -532,6 +564,35 @@ __global__ __launch_bounds__(256, 2) void generate_mixed_kernel(VolumeView<T> vo
     // the first increment of t and the grid's phase per unit of t
     const float ds0 = (t + s) - t;
     const double ptid = (double)pi_trange_inv;
+
+    // S = 4: the lane's nodes first .. until - 1 of 0 .. nodes (its sums are
+    // those nodes' terms), begun at the node before; t_back is t four nodes
+    // before the first, where the first finished weight belongs
+    int first = 0, until = 0, last_node = 0;
+    float t_back = t_near;
+    if constexpr (S == 4)
+    {
+        for (float tt = t_near; tt + s < t_far; tt += s)
+            ++last_node;
+        const int per = (last_node + 4) / 4;
+        first = quad * per;
+        until = min(first + per, last_node + 1);
+        if (first <= last_node && first > 0)
+        {
+            for (int i = 0; i < first - 1; ++i)
+            {
+                if (i == first - 4)
+                    t_back = t;
+                t += s;
+            }
+            if (first > 1)
+            {
+                p_prev = (double)(float)((double)((t - t_near) * pi_trange_inv) - kPi);
+                f_prev = (double)sample_at(vol, r, t, a);
+            }
+            ns = first;
+        }
+    }
 
     issue_at(pending, fminf(t + s, t_far));
     // advances to the next sample and to the terms of the node behind it; the
@@ -595,7 +656,15 @@ __global__ __launch_bounds__(256, 2) void generate_mixed_kernel(VolumeView<T> vo
         const double rstep = 1.0 / step, rstep2 = rstep * rstep;
         double rs, rc, zs, zc, js, jc, kr = 0.0, ki = 0.0;
         sincos_small(step, rs, rc);
-        sincos_small(-kPi - 4.0 * step, zs, zc);
+        if constexpr (S == 4)
+        {
+            td = t_back;
+            sincos_small(first >= 4 ? fma((double)t_back - (double)t_near, ptid, -kPi)
+                                    : (double)(first - 4) * step - kPi,
+                         zs, zc);
+        }
+        else
+            sincos_small(-kPi - 4.0 * step, zs, zc);
         if constexpr (CHUNK)
         {
             sincos_small(j0d * step, js, jc);
@@ -644,7 +713,19 @@ __global__ __launch_bounds__(256, 2) void generate_mixed_kernel(VolumeView<T> vo
         };
         double eps = p_prev + kPi; // of node 0, at q_0 = -pi
         int it = 0;
-        while (t + s < t_far) // t advances by s (1 - 2^-11) or more
+        if constexpr (S == 4)
+        {
+            it = first;
+            if (first > 0 && first <= last_node)
+            {
+                // the segment that ends at the first node: its left slope
+                double d, cp, cpp, shift;
+                segment(eps, d, cp, cpp, shift);
+                eps = p_prev - fma((double)t - (double)t_near, ptid, -kPi);
+                trap = 0.0;
+            }
+        }
+        while (S == 4 ? it < min(until, last_node) : t + s < t_far) // t advances by s (1 - 2^-11) or more
         {
             double d, cp, cpp, shift;
             segment(eps, d, cp, cpp, shift);
@@ -658,22 +739,70 @@ __global__ __launch_bounds__(256, 2) void generate_mixed_kernel(VolumeView<T> vo
             else
                 turn();
         }
-        double d, cp;
-        last_segment(eps, d, cp);
-        add(ring.push(d, 0.0, cp * rstep));
-        // the nodes whose weights are still pending: real ones up to the
-        // last, then the grid continued
-        const int nodes = ns - 2; // index of the last node
-        for (int i = 0; i < 8; ++i)
+        if constexpr (S == 4)
         {
-            if (nodes - 4 + i >= 0 && i < 4)
-                turn_real();
+            const bool last = first <= last_node && until > last_node;
+            if (last)
+            {
+                double d, cp;
+                last_segment(eps, d, cp);
+                add(ring.push(d, 0.0, cp * rstep));
+            }
+            if (first <= last_node)
+            {
+                // node of the phasor and of the ring's first pending weight
+                // (turned already behind a push of the loop)
+                int node = it - 4;
+                for (int i = 0; i < 8; ++i)
+                {
+                    if (i > 0 || last)
+                    {
+                        if (node >= 0 && node < last_node)
+                            turn_real();
+                        else
+                            turn();
+                        ++node;
+                    }
+                    add(ring.pop());
+                }
+            }
             else
-                turn();
-            add(ring.pop());
-        }
-        if constexpr (!CHUNK)
+                ns = 0;
+            auto quad_sum = [](double v) {
+                v += dpp_quad<0xB1>(v);
+                return v + dpp_quad<0x4E>(v);
+            };
+            g_left = quad_sum(last ? g_left : 0.0);
+            trap = quad_sum(trap);
+#pragma unroll
+            for (int j = 0; j < M; ++j)
+                sc[j] = quad_sum(sc[j]);
+            lo = fminf(lo, dpp_quad<0xB1>(lo));
+            lo = fminf(lo, dpp_quad<0x4E>(lo));
+            hi = fmaxf(hi, dpp_quad<0xB1>(hi));
+            hi = fmaxf(hi, dpp_quad<0x4E>(hi));
+            ns = last_node + 2;
             untangle_sums<M>(sc);
+        }
+        else
+        {
+            double d, cp;
+            last_segment(eps, d, cp);
+            add(ring.push(d, 0.0, cp * rstep));
+            // the nodes whose weights are still pending: real ones up to the
+            // last, then the grid continued
+            const int nodes = ns - 2; // index of the last node
+            for (int i = 0; i < 8; ++i)
+            {
+                if (nodes - 4 + i >= 0 && i < 4)
+                    turn_real();
+                else
+                    turn();
+                add(ring.pop());
+            }
+            if constexpr (!CHUNK)
+                untangle_sums<M>(sc);
+        }
     }
     else
     {
@@ -812,7 +941,7 @@ __global__ __launch_bounds__(256, 2) void generate_mixed_kernel(VolumeView<T> vo
                 sm2 = sm1;
                 sm1 = n;
             }
-            if (j >= 1 && j < jend)
+            if (j >= 1 && j < jend && (S == 1 || (j & 3) == quad))
                 mo[j] = (float)((sc[i] / (jd * jd) - (double)f_first * sj / jd) * norm);
         }
     }
@@ -831,6 +960,11 @@ __global__ __launch_bounds__(256, 2) void generate_mixed_kernel(VolumeView<T> vo
 // ---------------------------------------------------------------------------
 // launchers
 // ---------------------------------------------------------------------------
+// images of few rays take four lanes per ray: up to two wavefronts of 16 rays,
+// which is what the registers hold, on each of the 1024 SIMDs (192 x 160 rays:
+// 66 us by one lane, 44 by four; 256 x 192: 68 and 68; 256 x 256: 70 and 83)
+constexpr uint64_t kFewRays = 32768;
+
 // one launch of generate_mixed_kernel over `chunks` rows of blockIdx.y
 template <typename T, int M, bool CHUNK, bool GRID, int J0C>
 static void launch_mixed_kernel(const VolumeView<T> &v, const DevCamera &c, const GenArgs &a, float *o, uint32_t *b,
@@ -877,6 +1011,42 @@ static void launch_mixed(const VolumeView<T> &v, const DevCamera &c, const GenAr
         else if (chunks > 1)
             launch_mixed_kernel<T, M, true, GRID, 0>(v, c, a, o, b, s, rr, st, blocks, chunks - 1);
     }
+}
+
+// the gridded march by four lanes per ray; false if this call doesn't take it
+template <typename T>
+static bool launch_few_rays(const VolumeView<T> &v, const DevCamera &c, const GenArgs &a, float *o, uint32_t *b,
+                            int32_t *s, hipStream_t st)
+{
+    if constexpr (!std::is_same<T, SphParticle>::value)
+    {
+        if (a.m > 56 || (uint64_t)a.W * (uint64_t)a.H > kFewRays || !offsets_fit(v.nx, v.ny, v.nz, sizeof(T)))
+            return false;
+        const bool pow2 = exact_pow2(v.dmax.x - v.dmin.x) && exact_pow2(v.dmax.y - v.dmin.y) &&
+                          exact_pow2(v.dmax.z - v.dmin.z) && exact_pow2(a.data_max - a.data_min);
+        const dim3 grid((uint32_t)(((a.W + 7) / 8) * ((a.H + 7) / 8)));
+        float2 *none = nullptr;
+#define MRAY_FEW_CASE(MM)                                                                                             \
+    if (a.m <= MM)                                                                                                    \
+    {                                                                                                                 \
+        if (pow2)                                                                                                     \
+            hipLaunchKernelGGL((generate_mixed_kernel<T, MM, true, true, false, true, 0, 4>), grid, dim3(256), 0, st, \
+                               v, c, a, o, b, s, none);                                                               \
+        else                                                                                                          \
+            hipLaunchKernelGGL((generate_mixed_kernel<T, MM, true, false, false, true, 0, 4>), grid, dim3(256), 0,    \
+                               st, v, c, a, o, b, s, none);                                                           \
+        return true;                                                                                                  \
+    }
+        MRAY_FEW_CASE(8)
+        MRAY_FEW_CASE(16)
+        MRAY_FEW_CASE(24)
+        MRAY_FEW_CASE(30)
+        MRAY_FEW_CASE(40)
+        MRAY_FEW_CASE(50)
+        MRAY_FEW_CASE(56)
+#undef MRAY_FEW_CASE
+    }
+    return false;
 }
 
 template <typename T, bool GRID>
@@ -943,9 +1113,12 @@ static int dispatch_mixed(const VolumeView<T> &v, const DevCamera &c, const GenA
     g.rays = kRaysAll;
     if (rr || !((float)(a.m - 1) * (float)kPi * (a.step / longest) <= 1.01f))
         return dispatch_widths<T, false>(v, c, g, o, b, s, rr, st, blocks);
-    const int rc = dispatch_widths<T, true>(v, c, g, o, b, s, rr, st, blocks);
-    if (rc != 0)
-        return rc;
+    if (!launch_few_rays(v, c, g, o, b, s, st))
+    {
+        const int rc = dispatch_widths<T, true>(v, c, g, o, b, s, rr, st, blocks);
+        if (rc != 0)
+            return rc;
+    }
     const int axes = (d.x != 0.0f) + (d.y != 0.0f) + (d.z != 0.0f);
     if (c.orthographic && axes == 1)
     {

@@ -56,3 +56,45 @@ def test_gridded_march_matches_node_sums(name, dtype):
     assert bool((size > 0).any())
     bound = 2.0 ** -23 * size + 4e-8
     assert bool((d <= bound).all()), f"{name}: {float((d / bound).max()):.2f} of the bound"
+
+
+def _check(name, vol, cam, gp, W, H, m):
+    rr = torch.empty((H * W, 2), dtype=torch.float32, device="cuda")
+    ref, b_ref, s_ref = hip.generate(vol, cam, gp, W, H, m, ray_range=rr, want_samples=True)
+    mo, b, s = hip.generate(vol, cam, gp, W, H, m, want_samples=True)
+    assert torch.equal(b, b_ref) and torch.equal(s, s_ref)
+    d = (mo.double() - ref.double()).view(-1, m).abs().amax(1)
+    size = ref.double().view(-1, m).abs().amax(1)
+    bound = 2.0 ** -23 * size + 4e-8  # as above
+    assert bool((d <= bound).all()), f"{name}: {float((d / bound).max()):.2f} of the bound"
+
+
+# Images of few rays take four lanes per ray, so the cases above are theirs; the
+# same rays' lengths in images of many rays, which take one lane.
+@pytest.mark.parametrize("dtype", ["f32", "u8"])
+@pytest.mark.parametrize("name", ["resolved", "limit", "persp_mixed", "increments", "oblong", "two"])
+def test_gridded_march_many_rays(name, dtype):
+    n, (lo, hi), cam, W, H, m, step = CASES[name]
+    vol = synth.marschner_lobb(n) if lo < 0 else synth.mixing_layer(n, width=0.05)
+    v = torch.from_numpy(vol).cuda()
+    if dtype == "u8":
+        v = (v.clamp(0, 1) * 255).to(torch.uint8)
+    vol = hip.Volume(v, (lo,) * 3, (hi,) * 3)
+    gp = GenParams(step_size=step, transform_to_bounds=1, transform_bound_eps=0.01, compact_image=0,
+                   prediction_coding=0, bias=1e-4)
+    _check(name, vol, cam, gp, 261, 259, m)
+
+
+# rays of 1 to 17 nodes: lanes without a node, of one, of a ragged last share;
+# nodes fewer than the stencils are wide
+@pytest.mark.parametrize("nodes", range(1, 18))
+@pytest.mark.parametrize("cam", ["ortho", "persp"])
+def test_gridded_march_few_nodes(nodes, cam):
+    v = torch.from_numpy(synth.mixing_layer(24, width=0.3)).cuda()
+    vol = hip.Volume(v, (0,) * 3, (1,) * 3)
+    c = (synth.ortho_camera(pos=(0.5, 0.5, -1.0), right=(0.6, 0, 0), up=(0, 0.4, 0)) if cam == "ortho"
+         else synth.perspective_camera(fov_half_deg=12.0))
+    for m in (1, 2, 3, 4):
+        gp = GenParams(step_size=1.0 / (nodes + 0.5), transform_to_bounds=1, transform_bound_eps=0.01,
+                       compact_image=0, prediction_coding=0, bias=1e-4)
+        _check(f"{nodes} nodes, {m} moments", vol, c, gp, 21, 13, m)
