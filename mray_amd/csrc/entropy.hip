@@ -11,22 +11,24 @@
 //     ballot which of them carry a symbol;
 //   - the interval arithmetic is one serial chain per stream: every lane runs
 //     it on the same values (the symbol's model bounds broadcast from its
-//     lane with readlane), lane 0 writes the code bytes and propagates carries;
-//   - the model lives in LDS as counts and their exclusive running sums
-//     (d(k) = sum_{i<k} count_i / total is formed as (1 / total) * sum, the
-//     product the reference stores); its periodic update is a wave-wide scan.
+//     lane with readlane); the code leaves as 16-bit digits through a ring in
+//     LDS, 64 at a time (Encoder);
+//   - the model's counts and their exclusive running sums are in LDS (d(k) =
+//     sum_{i<k} count_i / total is formed as (1 / total) * sum, the product the
+//     reference stores); its periodic update is a wave-wide scan.
 //     The encoder looks up a run of symbols at once: the model is constant
 //     between updates, whose positions are known in advance;
-//   - the decoder finds a symbol's interval by testing 64 candidates at once:
+//   - the decoder finds a symbol's interval by testing many candidates at once:
 //     the interval ends base + length d(k) increase strictly with k (d grows
 //     by at least 2^-17 per symbol and length exceeds 2^-16, so the gaps are
 //     far above double rounding), so the largest k with
 //     base + length d(k) <= value + 2^-48 is the symbol the reference's
-//     bisection finds. A table over the model's cumulative counts (rebuilt at
-//     each model update) gives a symbol at or below it from a float estimate
-//     of the count at the value, and within 64 of it, so one test of 64
-//     candidates usually settles it; the code bytes come from a 256-byte
-//     window held in the wavefront's registers.
+//     bisection finds. Up to 2^11 symbols every lane tests its own share of the
+//     alphabet, with d in registers (LaneModel). Above, a table over the model's
+//     cumulative counts (rebuilt at each model update) gives a symbol at or
+//     below it from a float estimate of the count at the value, and within 64
+//     of it, so one test of 64 candidates usually settles it; the code bytes
+//     come from a 256-byte window held in the wavefront's registers.
 // All double arithmetic is unfused and correctly rounded (-ffp-contract=off),
 // in the reference's order, so codes and decoded values are bit-identical.
 #include <hip/hip_runtime.h>
