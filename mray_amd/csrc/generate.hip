@@ -33,6 +33,7 @@
 #include "cheb_blocks.hpp"
 #include "device_common.hpp"
 #include "launch.hpp"
+#include "march_grid.hpp"
 #include "sph_common.hpp"
 #include <type_traits>
 
@@ -420,7 +421,7 @@ template <int CTRL> __device__ __forceinline__ double dpp_quad(double v)
 // cosine, sine and weight recurrences and two sums). The stencils reach past
 // the ray's ends: c is defined there too. This needs the largest order
 // resolved by the grid, (m - 1) dphi <= 1 (at 1: 1.6e-3 of cp's terms, i.e.
-// ~1e-10 of the moments), and t's float increments uniform (t_far <= 8192 s:
+// ~1e-10 of the moments), and t's float increments uniform (|t| <= 8192 s:
 // where t passes a power of two they change by at most 2^-11): grid_resolves.
 // The wavefronts with a ray that fails it (a few samples for many moments)
 // are summed node by node (!GRID): the terms at p_k itself, cosine sums in
@@ -452,11 +453,6 @@ template <int CTRL> __device__ __forceinline__ double dpp_quad(double v)
 // 7.1 ms gridded (8.1 before the corners came in pairs); 2048 x 2048 x 1920
 // u8, 2048 x 2048 rays, 100 moments: 132 and 76 ms (the bytes' divisions and
 // the corner addresses are a third of that gain). Bound by VALU issue, then by load latency at two wavefronts per SIMD.
-__device__ __forceinline__ bool grid_resolves(int m, float dphi, float t_near, float t_far, float s)
-{
-    return (float)(m - 1) * dphi <= 1.0f && t_far <= 8192.0f * s && t_near + s < t_far;
-}
-
 template <typename T, int M, bool OFF32, bool POW2, bool CHUNK, bool GRID, int J0C, int S = 1>
 __global__ __launch_bounds__(256, 2) void generate_mixed_kernel(VolumeView<T> vol, DevCamera cam, GenArgs a,
                                                              float *__restrict__ out, uint32_t *__restrict__ bounds,
@@ -1133,8 +1129,10 @@ static int dispatch_mixed(const VolumeView<T> &v, const DevCamera &c, const GenA
         const float ru = d.x != 0.0f ? fabsf(c.right.x) + fabsf(c.up.x)
                          : d.y != 0.0f ? fabsf(c.right.y) + fabsf(c.up.y)
                                        : fabsf(c.right.z) + fabsf(c.up.z);
-        if (ru == 0.0f && from / len > c.znear && (float)(a.m - 1) * (float)kPi * (a.step / along) <= 0.99f &&
-            (from / len + along) * 1.01f <= 8192.0f * a.step && a.step < 0.5f * along)
+        // (from < 0: a camera inside or behind the box with a negative znear)
+        if (ru == 0.0f && from / len > c.znear && from >= 0.0f &&
+            (float)(a.m - 1) * (float)kPi * (a.step / along) <= 0.99f &&
+            (from / len + along) * 1.01f <= kGridReach * a.step && a.step < 0.5f * along)
             return 0;
     }
     g.rays = kRaysUngridded;
