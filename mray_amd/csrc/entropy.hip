@@ -37,6 +37,7 @@
 #include <vector>
 
 #include "device_common.hpp"
+#include "fastac_lanes.hpp"
 #include "launch.hpp"
 
 namespace mray
@@ -604,9 +605,8 @@ struct Decoder
 };
 
 // The model with its distribution in registers, for alphabets of up to 2^8
-// symbols (R = 1, 2, 4 symbols per lane): lane i holds d(iR) .. d(iR + R),
-// infinity from the alphabet's end on (such a symbol never qualifies), d(A) as
-// 1 (base + length * 1 is the reference's base + length).
+// symbols (R = 1, 2, 4 symbols per lane): lane i holds d(iR) .. d(iR + R) as
+// lane_dist gives them.
 // Above (R = 0, up to 2^11 symbols) the lanes hold the 64 block starts and the
 // block's at most 32 ends are read from LDS (dist).
 template <int R> struct LaneModel
@@ -645,7 +645,7 @@ template <int R> struct LaneModel
             for (int r = 0; r <= R; ++r)
             {
                 const uint32_t k = k0 + (uint32_t)r;
-                d[r] = (k < A) ? scale * (double)run : (r == R && k == A) ? 1.0 : __builtin_inf();
+                d[r] = lane_dist(k, A, scale * (double)run, r == R);
                 if (r < R && k < A)
                     run += count[k];
             }
@@ -744,35 +744,22 @@ struct LaneDecoder
         double x, y;
         if constexpr (R > 0)
         {
-            double z[R + 1];
-#pragma unroll
-            for (int r = 0; r <= R; ++r)
-                z[r] = base + length * M.d[r];
+            const LaneOffer o = lane_offer<R>(M.d, base, length, sv);
             // with none qualifying symbol 0, as the reference's bisection
-            const int j = last_of_prefix(!(z[0] > sv));
-            double xl = z[0], yl = z[1];
-            uint32_t sub = 0;
-#pragma unroll
-            for (int r = 1; r < R; ++r)
-            {
-                const bool q = !(z[r] > sv);
-                xl = q ? z[r] : xl;
-                yl = q ? z[r + 1 <= R ? r + 1 : R] : yl;
-                sub = q ? (uint32_t)r : sub;
-            }
-            x = readlane_f64(xl, j);
-            y = readlane_f64(yl, j);
+            const int j = last_of_prefix(o.any);
+            x = readlane_f64(o.x, j);
+            y = readlane_f64(o.y, j);
             s = (uint32_t)j * R;
             if constexpr (R > 1)
-                s += (uint32_t)__builtin_amdgcn_readlane((int)sub, j);
+                s += (uint32_t)__builtin_amdgcn_readlane((int)o.sub, j);
         }
         else
         {
             const double zc = base + length * M.d[0];
             const uint32_t n = M.A / 64u, i = min((uint32_t)threadIdx.x, n);
-            const uint32_t k0 = (uint32_t)last_of_prefix(!(zc > sv)) << M.shift;
+            const uint32_t k0 = (uint32_t)last_of_prefix(candidate(zc, sv)) << M.shift;
             const double z = base + length * M.dist[k0 + i];
-            const int j = last_of_prefix(!(z > sv), (1ull << n) - 1ull);
+            const int j = last_of_prefix(candidate(z, sv), (1ull << n) - 1ull);
             x = readlane_f64(z, j);
             y = readlane_f64(z, j + 1);
             s = k0 + (uint32_t)j;

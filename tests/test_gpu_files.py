@@ -100,6 +100,24 @@ def test_entropy_matches_oracle(hipmod, W, H, m, pc, width, empty):
         assert np.array_equal(dec.view(np.uint32), requantized(O, data, index, pc, bits).view(np.uint32))
 
 
+@pytest.mark.parametrize("width,symbols", [(5, 1400000), (1, 70000), (7, 400000), (9, 50000)])
+def test_entropy_malformed_code(hipmod, width, symbols):
+    """Codes of 0xFF bytes leave the coder's interval (at 5 and 7 bits until the
+    code's value is infinite): the same values as the reference's bisection
+    decodes, within the alphabet."""
+    W, H, m = symbols // 50, 50, 2
+    index = (2 * np.arange(W * H + 1)).astype(np.uint32)
+    bits = np.array([10, width], np.uint8)
+    code = np.full(1 << 20, 255, np.uint8)
+    sec = np.concatenate([np.array([W * H], np.uint32).view(np.uint8), np.zeros(2 * W * H, np.uint8),
+                          np.array([len(code)], np.uint32).view(np.uint8), code])
+    ref = Oracle().entropy_decode(W, H, m, sec, index, 1, bits)
+    print(f"[entropy] malformed, {width} bits", flush=True)
+    dec = hipmod.entropy_decode(sec, dev(index.view(np.int32)), W, H, m, 1, bits).cpu().numpy()
+    assert np.array_equal(dec.view(np.uint32), ref.view(np.uint32))
+    assert dec.min() >= 0.0 and dec.max() <= 1.0
+
+
 def test_entropy_rejects_bad_widths(hipmod):
     index = np.array([0, 2, 4], np.uint32)
     data = np.zeros(4, np.float32)
