@@ -341,56 +341,6 @@ __device__ __forceinline__ void accumulate_node_chunk_c(double (&sc)[M], float (
     }
 }
 
-// Pending weights of the eight grid nodes around the newest one (the 9-point
-// stencils of the first two derivatives, error (j Delta)^8 / 630 and / 3150 of
-// the term). push adds node k's functional d c + cp c' + cpp c'' and returns
-// the finished weight of node k - 4; A = cpp / Delta^2, B = cp / Delta. The
-// ring moves on by writing each sum into the next slot (no copies).
-struct WeightRing
-{
-    double w[8];
-
-    // r = a b + c with r a register of its own (left to the compiler, each
-    // sum is formed in its old slot's registers and copied over)
-    static __device__ __forceinline__ void fma_to(double &r, double a, double b, double c)
-    {
-        asm("v_fma_f64 %0, %1, %2, %3" : "=v"(r) : "s"(a), "v"(b), "v"(c));
-    }
-
-    __device__ __forceinline__ WeightRing()
-    {
-#pragma unroll
-        for (int i = 0; i < 8; ++i)
-            w[i] = 0.0;
-    }
-
-    __device__ __forceinline__ double push(double d, double A, double B)
-    {
-        constexpr double a0 = -205.0 / 72.0, a1 = 8.0 / 5.0, a2 = -1.0 / 5.0, a3 = 8.0 / 315.0, a4 = -1.0 / 560.0;
-        constexpr double b1 = 4.0 / 5.0, b2 = -1.0 / 5.0, b3 = 4.0 / 105.0, b4 = -1.0 / 280.0;
-        const double out = fma(a4, A, fma(-b4, B, w[0]));
-        fma_to(w[0], a3, A, fma(-b3, B, w[1]));
-        fma_to(w[1], a2, A, fma(-b2, B, w[2]));
-        fma_to(w[2], a1, A, fma(-b1, B, w[3]));
-        fma_to(w[3], a0, A, w[4] + d);
-        fma_to(w[4], a1, A, fma(b1, B, w[5]));
-        fma_to(w[5], a2, A, fma(b2, B, w[6]));
-        fma_to(w[6], a3, A, fma(b3, B, w[7]));
-        w[7] = fma(a4, A, b4 * B);
-        return out;
-    }
-
-    __device__ __forceinline__ double pop()
-    {
-        const double out = w[0];
-#pragma unroll
-        for (int i = 0; i < 7; ++i)
-            w[i] = w[i + 1];
-        w[7] = 0.0;
-        return out;
-    }
-};
-
 // a value of another lane of the quad (CTRL: quad_perm)
 template <int CTRL> __device__ __forceinline__ float dpp_quad(float v)
 {
@@ -422,7 +372,8 @@ template <int CTRL> __device__ __forceinline__ double dpp_quad(double v)
 // the ray's ends: c is defined there too. This needs the largest order
 // resolved by the grid, (m - 1) dphi <= 1 (at 1: 1.6e-3 of cp's terms, i.e.
 // ~1e-10 of the moments), and t's float increments uniform (|t| <= 8192 s:
-// where t passes a power of two they change by at most 2^-11): grid_resolves.
+// where t passes a power of two they change by at most 2^-11): grid_resolves;
+// GridStep has what a change next to 8192 s costs.
 // The wavefronts with a ray that fails it (a few samples for many moments)
 // are summed node by node (!GRID): the terms at p_k itself, cosine sums in
 // FP64 and the ulp-sized sine terms in FP32, five operations per moment. The
@@ -557,9 +508,11 @@ __global__ __launch_bounds__(256, 2) void generate_mixed_kernel(VolumeView<T> vo
     double f_prev = (double)f_first, p_prev = (double)phase0;
     double g_left = 0.0, w_left = 0.0;
     const double dphid = (double)dphi, rdphi = 1.0 / dphid;
-    // the first increment of t and the grid's phase per unit of t
-    const float ds0 = (t + s) - t;
+    // the grid's phase per unit of t, and its first step
     const double ptid = (double)pi_trange_inv;
+    GridStep step_at;
+    step_at.start((t + s) - t, ptid);
+    const float ds0 = step_at.ds;
 
     // S = 4: the lane's nodes first .. until - 1 of 0 .. nodes (its sums are
     // those nodes' terms), begun at the node before; t_back is t four nodes
@@ -594,15 +547,13 @@ __global__ __launch_bounds__(256, 2) void generate_mixed_kernel(VolumeView<T> vo
     // advances to the next sample and to the terms of the node behind it; the
     // last segment [p_K, 0] (src/raymarch_generate.h:107-114) starts exactly
     // at p_K and its line ends exactly at its sample
-    float ds = ds0; // t's last increment
     auto segment = [&](double eps, double &d, double &cp, double &cpp, double &shift) {
         const float tn = t + s, dn = tn - t;
         shift = 0.0;
-        if (dn != ds)
+        if (dn != step_at.ds)
         {
             asm volatile(""); // rare: a branch, not a select of its result
-            shift = ((double)dn - (double)ds) * ptid;
-            ds = dn;
+            shift = step_at.change(dn, ptid);
         }
         t = tn;
         const float p = (float)((double)((t - t_near) * pi_trange_inv) - kPi);
@@ -649,7 +600,6 @@ __global__ __launch_bounds__(256, 2) void generate_mixed_kernel(VolumeView<T> vo
         WeightRing ring;
         float dsd = ds0, td = t_near;
         double step = (double)ds0 * ptid;
-        const double rstep = 1.0 / step, rstep2 = rstep * rstep;
         double rs, rc, zs, zc, js, jc, kr = 0.0, ki = 0.0;
         sincos_small(step, rs, rc);
         if constexpr (S == 4)
@@ -726,10 +676,8 @@ __global__ __launch_bounds__(256, 2) void generate_mixed_kernel(VolumeView<T> vo
             double d, cp, cpp, shift;
             segment(eps, d, cp, cpp, shift);
             eps = p_prev - fma((double)t - (double)t_near, ptid, -kPi);
-            const double A = cpp * rstep2;
-            // where the grid's step changes by `shift` behind this node, the
-            // second difference picks up a first one
-            add(ring.push(d, A, fma(-1.2690476190476190 * A, shift, cp) * rstep));
+            const double A = step_at.second(cpp);
+            add(ring.push(d, A, step_at.first(cp, A, shift)));
             if (it++ >= 4)
                 turn_real();
             else
@@ -742,7 +690,7 @@ __global__ __launch_bounds__(256, 2) void generate_mixed_kernel(VolumeView<T> vo
             {
                 double d, cp;
                 last_segment(eps, d, cp);
-                add(ring.push(d, 0.0, cp * rstep));
+                add(ring.push(d, 0.0, cp * step_at.rstep));
             }
             if (first <= last_node)
             {
@@ -784,7 +732,7 @@ __global__ __launch_bounds__(256, 2) void generate_mixed_kernel(VolumeView<T> vo
         {
             double d, cp;
             last_segment(eps, d, cp);
-            add(ring.push(d, 0.0, cp * rstep));
+            add(ring.push(d, 0.0, cp * step_at.rstep));
             // the nodes whose weights are still pending: real ones up to the
             // last, then the grid continued
             const int nodes = ns - 2; // index of the last node
