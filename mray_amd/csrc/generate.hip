@@ -49,15 +49,6 @@ struct GenArgs
     int transform_to_bounds;
     int compact_image;
     float bound_eps;
-    int rays; // which rays a launch of generate_mixed_kernel takes (GenRays)
-};
-
-// the rays of a MIXED launch, by wavefront: every one, or those summed node by
-// node where another launch takes the gridded ones
-enum GenRays : int
-{
-    kRaysAll = 0,
-    kRaysUngridded = 1,
 };
 
 // Sample at t along r (origin + t * dir in float, as the reference).
@@ -375,10 +366,13 @@ template <int CTRL> __device__ __forceinline__ double dpp_quad(double v)
 // where t passes a power of two they change by at most 2^-11): grid_resolves;
 // GridStep has what a change next to 8192 s costs.
 // The wavefronts with a ray that fails it (a few samples for many moments)
-// are summed node by node (!GRID): the terms at p_k itself, cosine sums in
-// FP64 and the ulp-sized sine terms in FP32, five operations per moment. The
-// two are kernels of their own, launched over the same tiles (registers: the
-// sine sums would cost the gridded march a wavefront per SIMD at 30 moments).
+// are summed node by node: the terms at p_k itself, cosine sums in FP64 and
+// the ulp-sized sine terms in FP32, five operations per moment. GRID: each
+// wavefront takes the form its rays allow, in one launch, so that neither form
+// waits for the other's last wavefronts (128^3 f32 from a perspective camera,
+// 50 moments, 256 steps: 512 x 512 rays 522 us as two launches over the same
+// tiles, 499 all node by node, 364 in one; 90 x 70 rays 322, 266 and 240).
+// !GRID: node by node throughout.
 //
 // A pass that records the rays' normalisation is the forward of a gradient
 // (generate_backward) and is summed node by node for every ray: the bounded
@@ -392,11 +386,12 @@ template <int CTRL> __device__ __forceinline__ double dpp_quad(double v)
 // image of m > M: it writes moments 0 .. M - 1, the bounds, the ray range and
 // the sample counts); the CHUNK kernel runs the later ones,
 // j0 = (blockIdx.y + 1) M.
-// J0C: a chunk start known at compile time (!GRID).
+// J0C: a chunk start known at compile time.
 // S = 4: four lanes per ray, each the terms of a quarter of its nodes (from the
 // segment that ends at the first of them to the one that starts at the last),
 // their sums added at the end. For images of few rays, which leave most SIMDs
-// without a wavefront: a lone wavefront takes 0.5 us per node.
+// without a wavefront: a lone wavefront takes 0.5 us per node. A tile that is
+// summed node by node leaves three of its wavefronts without work.
 // Measured (128^3, 30 moments): 100 steps, up to 16384 rays 62 us by one lane,
 // 28 by four; 1000 steps 541 and 179 (each lane first adds up its t).
 //
@@ -404,8 +399,18 @@ template <int CTRL> __device__ __forceinline__ double dpp_quad(double v)
 // 7.1 ms gridded (8.1 before the corners came in pairs); 2048 x 2048 x 1920
 // u8, 2048 x 2048 rays, 100 moments: 132 and 76 ms (the bytes' divisions and
 // the corner addresses are a third of that gain). Bound by VALU issue, then by load latency at two wavefronts per SIMD.
+// wavefronts per SIMD a kernel's registers are held to. Up to 30 moments (28 in
+// general domains) a GRID kernel comes to 168 to 184 without a bound, and 3 to 14
+// of them spilled cost less than the third wavefront is worth (128^3 f32, 509 x
+// 387 rays, 30 moments: 350 us by two, 320 by three; in a domain of 0.9^3 396
+// and 422).
+template <int M, bool POW2, bool GRID, int S> constexpr int mixed_wavefronts()
+{
+    return !GRID ? 1 : (S == 1 && M <= (POW2 ? 30 : 28)) ? 3 : 2;
+}
+
 template <typename T, int M, bool OFF32, bool POW2, bool CHUNK, bool GRID, int J0C, int S = 1>
-__global__ __launch_bounds__(256, 2) void generate_mixed_kernel(VolumeView<T> vol, DevCamera cam, GenArgs a,
+__global__ __launch_bounds__(256, (mixed_wavefronts<M, POW2, GRID, S>())) void generate_mixed_kernel(VolumeView<T> vol, DevCamera cam, GenArgs a,
                                                              float *__restrict__ out, uint32_t *__restrict__ bounds,
                                                              int32_t *__restrict__ samples,
                                                              float2 *__restrict__ ray_range)
@@ -433,20 +438,28 @@ __global__ __launch_bounds__(256, 2) void generate_mixed_kernel(VolumeView<T> vo
     bool tile_gridded = false;
     if constexpr (S == 4)
     {
-        // whether the tile's rays are gridded: as its wavefront decides in the
-        // other launch
+        // whether the tile's rays are gridded: as its wavefront decides with
+        // one lane per ray
         const bool inside = x < a.W && y < a.H;
         const float step_phase = (float)(kPi * (double)(a.step / (t_far - t_near)));
         tile_gridded = !__syncthreads_or(inside && hit && t_far > 0 && !grid_resolves(m, step_phase, t_near, t_far, a.step));
-        if (!inside)
+        if (!tile_gridded)
+        {
+            // one wavefront of the tile's 64 rays, as with one lane per ray
+            if (tid >= 64)
+                return;
+            tile_pixel(tile, a.W, lane, x, y);
+            r = pixel_ray(cam, a.W, a.H, x, y);
+            hit = intersect_aabb(r, vol.dmin, vol.dmax, t_near, t_far);
+            t_near = rmax(t_near, cam.znear);
+        }
+        if (x >= a.W || y >= a.H)
             return;
     }
     size_t pix = (size_t)y * a.W + x;
     float *mo = out + pix * (size_t)m;
     if (!(hit && (t_far > 0)))
     {
-        if (!GRID && a.rays == kRaysUngridded)
-            return; // written by the gridded launch
         if (!(a.transform_to_bounds && a.compact_image))
             for (int j = j0; j < jend; ++j)
                 mo[j] = 0.f;
@@ -466,9 +479,10 @@ __global__ __launch_bounds__(256, 2) void generate_mixed_kernel(VolumeView<T> vo
     const float pi_trange_inv = (float)(kPi / (double)(t_far - t_near));
     const float dphi = (float)(kPi * (double)(s / (t_far - t_near)));
     // by wavefront: whether its rays are gridded
-    const bool gridded = S == 4 ? tile_gridded : !__any(!grid_resolves(m, dphi, t_near, t_far, s));
-    if (GRID ? !gridded : (gridded && a.rays == kRaysUngridded))
-        return;
+    bool gridded = false;
+    if constexpr (GRID)
+        gridded = S == 4 ? tile_gridded : __ballot(!grid_resolves(m, dphi, t_near, t_far, s)) == 0ull;
+    const bool one_lane = S == 1 || !gridded;
 
     float t = t_near;
     const float f_first = sample_at(vol, r, t, a);
@@ -519,7 +533,7 @@ __global__ __launch_bounds__(256, 2) void generate_mixed_kernel(VolumeView<T> vo
     // before the first, where the first finished weight belongs
     int first = 0, until = 0, last_node = 0;
     float t_back = t_near;
-    if constexpr (S == 4)
+    if (!one_lane)
     {
         for (float tt = t_near; tt + s < t_far; tt += s)
             ++last_node;
@@ -543,14 +557,13 @@ __global__ __launch_bounds__(256, 2) void generate_mixed_kernel(VolumeView<T> vo
         }
     }
 
-    issue_at(pending, fminf(t + s, t_far));
     // advances to the next sample and to the terms of the node behind it; the
     // last segment [p_K, 0] (src/raymarch_generate.h:107-114) starts exactly
     // at p_K and its line ends exactly at its sample
-    auto segment = [&](double eps, double &d, double &cp, double &cpp, double &shift) {
+    auto segment = [&](double eps, double &d, double &cp, double &cpp, double &shift) __attribute__((always_inline)) {
         const float tn = t + s, dn = tn - t;
         shift = 0.0;
-        if (dn != step_at.ds)
+        if (__builtin_expect(dn != step_at.ds, 0))
         {
             asm volatile(""); // rare: a branch, not a select of its result
             shift = step_at.change(dn, ptid);
@@ -580,7 +593,7 @@ __global__ __launch_bounds__(256, 2) void generate_mixed_kernel(VolumeView<T> vo
         p_prev = pd;
         ++ns;
     };
-    auto last_segment = [&](double eps, double &d, double &cp) {
+    auto last_segment = [&](double eps, double &d, double &cp) __attribute__((always_inline)) {
         const float f = density(pending.value());
         lo = rmin(lo, f);
         hi = rmax(hi, f);
@@ -593,8 +606,9 @@ __global__ __launch_bounds__(256, 2) void generate_mixed_kernel(VolumeView<T> vo
         ++ns;
     };
 
-    if constexpr (GRID)
+    if (GRID && gridded)
     {
+        issue_at(pending, fminf(t + s, t_far));
         // the phasor of the node whose weight is finished, four nodes behind,
         // turned by the grid's step; td is that node's t
         WeightRing ring;
@@ -616,7 +630,7 @@ __global__ __launch_bounds__(256, 2) void generate_mixed_kernel(VolumeView<T> vo
             sincos_small(j0d * step, js, jc);
             sincos_small(j0d * (-kPi - 4.0 * step), ki, kr);
         }
-        auto add = [&](double w) {
+        auto add = [&](double w) __attribute__((always_inline)) {
             // a weight of exactly zero (inside a stretch of zero density) adds
             // nothing; where every lane of the wavefront has one, skipped
             if (w != 0.0)
@@ -632,7 +646,7 @@ __global__ __launch_bounds__(256, 2) void generate_mixed_kernel(VolumeView<T> vo
                 }
             }
         };
-        auto turn = [&]() {
+        auto turn = [&]() __attribute__((always_inline)) {
             const double nc = fma(zc, rc, -zs * rs);
             zs = fma(zs, rc, zc * rs);
             zc = nc;
@@ -645,9 +659,9 @@ __global__ __launch_bounds__(256, 2) void generate_mixed_kernel(VolumeView<T> vo
         };
         // the turn to the next real node: t's increment changes where t
         // passes a power of two
-        auto turn_real = [&]() {
+        auto turn_real = [&]() __attribute__((always_inline)) {
             const float tn = td + s;
-            if (tn - td != dsd)
+            if (__builtin_expect(tn - td != dsd, 0))
             {
                 dsd = tn - td;
                 sincos_small((double)dsd * ptid, rs, rc);
@@ -712,7 +726,7 @@ __global__ __launch_bounds__(256, 2) void generate_mixed_kernel(VolumeView<T> vo
             }
             else
                 ns = 0;
-            auto quad_sum = [](double v) {
+            auto quad_sum = [](double v) __attribute__((always_inline)) {
                 v += dpp_quad<0xB1>(v);
                 return v + dpp_quad<0x4E>(v);
             };
@@ -750,6 +764,7 @@ __global__ __launch_bounds__(256, 2) void generate_mixed_kernel(VolumeView<T> vo
     }
     else
     {
+        issue_at(pending, fminf(t + s, t_far));
         float ss[M];
 #pragma unroll
         for (int j = 0; j < M; ++j)
@@ -760,7 +775,7 @@ __global__ __launch_bounds__(256, 2) void generate_mixed_kernel(VolumeView<T> vo
         double zs, zc, kc = 1.0, ks = 0.0, kc1, ks1;
         sincos_small((double)node_phase, zs, zc);
         bool turned = false; // kc, ks already are those of the node
-        auto chunk_start = [&](float ph) {
+        auto chunk_start = [&](float ph) __attribute__((always_inline)) {
             if constexpr (CHUNK)
             {
                 if (!turned)
@@ -770,7 +785,7 @@ __global__ __launch_bounds__(256, 2) void generate_mixed_kernel(VolumeView<T> vo
             }
         };
         chunk_start(node_phase);
-        auto add = [&](double d, double e, double h) {
+        auto add = [&](double d, double e, double h) __attribute__((always_inline)) {
             if constexpr (CHUNK && J0C > 0)
                 accumulate_node_chunk_c<M, J0C>(sc, ss, d, e, (float)h, zc, kc, (float)ks, kc1, (float)ks1);
             else if constexpr (CHUNK)
@@ -885,7 +900,7 @@ __global__ __launch_bounds__(256, 2) void generate_mixed_kernel(VolumeView<T> vo
                 sm2 = sm1;
                 sm1 = n;
             }
-            if (j >= 1 && j < jend && (S == 1 || (j & 3) == quad))
+            if (j >= 1 && j < jend && (one_lane || (j & 3) == quad))
                 mo[j] = (float)((sc[i] / (jd * jd) - (double)f_first * sj / jd) * norm);
         }
     }
@@ -941,8 +956,8 @@ static void launch_mixed_kernel(const VolumeView<T> &v, const DevCamera &c, cons
 }
 
 // `chunks` > 1 marches the moments in chunks of M: the unchunked kernel for
-// the first, then the later ones over blockIdx.y (or, summed node by node and
-// two, the second from j0 = M as a compile-time start)
+// the first, then the later ones over blockIdx.y (or, of two, the second from
+// j0 = M as a compile-time start)
 template <typename T, int M, bool GRID, bool CHUNK = false>
 static void launch_mixed(const VolumeView<T> &v, const DevCamera &c, const GenArgs &a, float *o, uint32_t *b,
                          int32_t *s, float2 *rr, hipStream_t st, uint32_t blocks, int chunks = 1)
@@ -950,14 +965,14 @@ static void launch_mixed(const VolumeView<T> &v, const DevCamera &c, const GenAr
     launch_mixed_kernel<T, M, false, GRID, 0>(v, c, a, o, b, s, rr, st, blocks, 1);
     if constexpr (CHUNK)
     {
-        if (chunks == 2 && !GRID)
-            launch_mixed_kernel<T, M, true, GRID, GRID ? 0 : M>(v, c, a, o, b, s, rr, st, blocks, 1);
+        if (chunks == 2)
+            launch_mixed_kernel<T, M, true, GRID, M>(v, c, a, o, b, s, rr, st, blocks, 1);
         else if (chunks > 1)
             launch_mixed_kernel<T, M, true, GRID, 0>(v, c, a, o, b, s, rr, st, blocks, chunks - 1);
     }
 }
 
-// the gridded march by four lanes per ray; false if this call doesn't take it
+// the march by four lanes per ray; false if this call doesn't take it
 template <typename T>
 static bool launch_few_rays(const VolumeView<T> &v, const DevCamera &c, const GenArgs &a, float *o, uint32_t *b,
                             int32_t *s, hipStream_t st)
@@ -985,7 +1000,9 @@ static bool launch_few_rays(const VolumeView<T> &v, const DevCamera &c, const Ge
         MRAY_FEW_CASE(16)
         MRAY_FEW_CASE(24)
         MRAY_FEW_CASE(30)
+        MRAY_FEW_CASE(36)
         MRAY_FEW_CASE(40)
+        MRAY_FEW_CASE(44)
         MRAY_FEW_CASE(50)
         MRAY_FEW_CASE(56)
 #undef MRAY_FEW_CASE
@@ -1037,54 +1054,25 @@ static int dispatch_widths(const VolumeView<T> &v, const DevCamera &c, const Gen
     return MRAY_ERR_UNSUPPORTED;
 }
 
-// The gridded march for the wavefronts whose rays the grid resolves, the march
-// summed node by node for the others: both launches, unless one is known to
-// have no wavefront. A pass that records the rays' normalisation (ray_range)
-// is summed node by node throughout (see the kernel), and so is an image whose
-// longest possible ray has too few samples for its moments; all rays of an
-// orthographic camera along an axis are as long as the box.
+// The kernel that lets each wavefront take the gridded march, unless none can:
+// a pass that records the rays' normalisation (ray_range) is summed node by
+// node throughout (see the kernel), and so is an image whose longest possible
+// ray has too few samples for its moments.
 template <typename T>
 static int dispatch_mixed(const VolumeView<T> &v, const DevCamera &c, const GenArgs &a, float *o, uint32_t *b,
                           int32_t *s, float2 *rr, hipStream_t st, uint32_t blocks)
 {
-    GenArgs g = a;
     const float ex = v.dmax.x - v.dmin.x, ey = v.dmax.y - v.dmin.y, ez = v.dmax.z - v.dmin.z;
     const Vec3 d = c.dir;
     // directions of perspective rays are unit vectors, an orthographic
     // camera's is as given
     const float len = c.orthographic ? sqrtf(d.x * d.x + d.y * d.y + d.z * d.z) : 1.0f;
     const float longest = sqrtf(ex * ex + ey * ey + ez * ez) / len;
-    g.rays = kRaysAll;
     if (rr || !((float)(a.m - 1) * (float)kPi * (a.step / longest) <= 1.01f))
-        return dispatch_widths<T, false>(v, c, g, o, b, s, rr, st, blocks);
-    if (!launch_few_rays(v, c, g, o, b, s, st))
-    {
-        const int rc = dispatch_widths<T, true>(v, c, g, o, b, s, rr, st, blocks);
-        if (rc != 0)
-            return rc;
-    }
-    const int axes = (d.x != 0.0f) + (d.y != 0.0f) + (d.z != 0.0f);
-    if (c.orthographic && axes == 1)
-    {
-        const float along = (d.x != 0.0f ? ex : d.y != 0.0f ? ey : ez) / len;
-        // from outside the box (znear cuts nothing off), with a margin for
-        // rounding, and not too many steps from the camera
-        const float from = d.x != 0.0f ? (d.x > 0 ? v.dmin.x - c.pos.x : c.pos.x - v.dmax.x)
-                           : d.y != 0.0f ? (d.y > 0 ? v.dmin.y - c.pos.y : c.pos.y - v.dmax.y)
-                                         : (d.z > 0 ? v.dmin.z - c.pos.z : c.pos.z - v.dmax.z);
-        // the slab's near end is at from / len for every pixel (right and up
-        // have no component along the axis)
-        const float ru = d.x != 0.0f ? fabsf(c.right.x) + fabsf(c.up.x)
-                         : d.y != 0.0f ? fabsf(c.right.y) + fabsf(c.up.y)
-                                       : fabsf(c.right.z) + fabsf(c.up.z);
-        // (from < 0: a camera inside or behind the box with a negative znear)
-        if (ru == 0.0f && from / len > c.znear && from >= 0.0f &&
-            (float)(a.m - 1) * (float)kPi * (a.step / along) <= 0.99f &&
-            (from / len + along) * 1.01f <= kGridReach * a.step && a.step < 0.5f * along)
-            return 0;
-    }
-    g.rays = kRaysUngridded;
-    return dispatch_widths<T, false>(v, c, g, o, b, s, rr, st, blocks);
+        return dispatch_widths<T, false>(v, c, a, o, b, s, rr, st, blocks);
+    if (launch_few_rays(v, c, a, o, b, s, st))
+        return 0;
+    return dispatch_widths<T, true>(v, c, a, o, b, s, rr, st, blocks);
 }
 
 // PLAIN keeps m floats per thread in LDS: 256-thread blocks while that fits
@@ -1685,7 +1673,6 @@ int launch_generate_adjoint(const float *vox, int nx, int ny, int nz, const floa
     a.transform_to_bounds = p.transform_to_bounds;
     a.compact_image = p.compact_image;
     a.bound_eps = p.transform_bound_eps;
-    a.rays = kRaysAll;
     DevCamera c = make_dev_camera(cam);
     const uint32_t ntiles = (uint32_t)(((W + 7) / 8) * ((H + 7) / 8));
     const uint32_t blocks = (ntiles + 3) / 4;
@@ -1759,7 +1746,6 @@ int launch_generate(const void *vox, int dtype, int nx, int ny, int nz, const fl
     a.transform_to_bounds = p.transform_to_bounds;
     a.compact_image = p.compact_image;
     a.bound_eps = p.transform_bound_eps;
-    a.rays = kRaysAll;
     DevCamera c = make_dev_camera(cam);
     uint32_t ntiles = (uint32_t)(((W + 7) / 8) * ((H + 7) / 8));
     uint32_t blocks = (ntiles + 3) / 4;

@@ -27,6 +27,8 @@ CASES = {
     "limit": (64, (-1, 1), synth.ortho_camera(), 16, 16, 41, 1.0 / 64),
     "past_limit": (64, (-1, 1), synth.ortho_camera(), 16, 16, 42, 1.0 / 64),
     "persp_mixed": (48, (0, 1), synth.perspective_camera(aspect=40 / 30), 40, 30, 24, 0.5 / 48),
+    # tiles of both forms, and ones whose rays differ, in one launch
+    "persp_edge": (64, (0, 1), synth.perspective_camera(aspect=9 / 7), 90, 70, 44, 0.5 / 64),
     "chunks2": (96, (0, 1), synth.perspective_camera(position=(0.45, 0.5, -0.9)), 19, 21, 61, 0.25 / 96),
     "chunks3": (96, (0, 1), synth.perspective_camera(), 16, 9, 101, 0.15 / 96),
     "increments": (80, (0, 1), synth.perspective_camera(position=(0.5, 0.5, -3.3), fov_half_deg=9.0), 24, 24, 33,
@@ -74,7 +76,7 @@ def _check(name, vol, cam, gp, W, H, m):
 # Images of few rays take four lanes per ray, so the cases above are theirs; the
 # same rays' lengths in images of many rays, which take one lane.
 @pytest.mark.parametrize("dtype", ["f32", "u8"])
-@pytest.mark.parametrize("name", ["resolved", "limit", "persp_mixed", "increments", "reach", "reach_chunks", "inside", "behind",
+@pytest.mark.parametrize("name", ["resolved", "limit", "persp_mixed", "persp_edge", "increments", "reach", "reach_chunks", "inside", "behind",
                                   "oblong", "two"])
 def test_gridded_march_many_rays(name, dtype):
     n, (lo, hi), cam, W, H, m, step = CASES[name]
