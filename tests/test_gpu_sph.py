@@ -124,3 +124,27 @@ def test_particle_march_matches_oracle(hip, O, form):
     assert errg.max() <= 2e-5
     pv.close()
 
+
+@pytest.mark.parametrize("W,H", [(14, 14), (200, 190)])
+@pytest.mark.parametrize("m", [8, 30, 60])
+def test_particle_march_is_summed_node_by_node(W, H, m):
+    """Every march of a particle set sums its moments node by node (the gridded
+    march's registers cost more than its sums give there): the same bits with
+    and without ray_range, for images of few and of many rays."""
+    import torch
+
+    from mray_amd import hip, synth
+    from mray_amd.types import GenParams
+
+    hip.init(0)
+    rng = np.random.default_rng(3)
+    p = [torch.from_numpy(rng.random(3000).astype(np.float32)).cuda() for _ in range(4)]
+    pv = hip.ParticleVolume(*p, 0.07, (0.0, 0.0, 0.0), (1.0, 1.0, 1.0))
+    cam = synth.perspective_camera()
+    gp = GenParams(step_size=0.004, transform_to_bounds=1, transform_bound_eps=0.01, compact_image=0,
+                   prediction_coding=0)
+    rr = torch.empty((H * W, 2), dtype=torch.float32, device="cuda")
+    a, _, _ = hip.generate(pv, cam, gp, W, H, m)
+    b, _, _ = hip.generate(pv, cam, gp, W, H, m, ray_range=rr)
+    assert torch.equal(a, b)
+    pv.close()
