@@ -301,12 +301,31 @@ __global__ __launch_bounds__(256) void reconstruct_mixed_kernel(DevCamera cam, R
     // entries, the surplus zeroed after), so that they are in flight together:
     // one conditional load and wait after another let L2 evict the rows'
     // cache lines between the loads (3.4x the multipliers' bytes from HBM)
+    // All of them are issued in the row's order before the first is used: among
+    // the coefficients' sums, which begin with the last, the loads spread out
+    // (1024 x 1024 rays, 30 moments: 141 us of the call, 48 now; FP64
+    // multipliers 232 and 50). Above 96 the registers don't hold a row in
+    // flight beside the multipliers (104, 512 x 512 rays: 321 us, 353 with it).
     double lam[M];
-#pragma unroll
-    for (int l = 0; l < M; ++l)
+    if constexpr (kTwoSteps<M>)
     {
-        const LagT v = lag[off + min(l, nm - 1)];
-        lam[l] = (l < nm) ? (l ? 2.0 : 1.0) * (double)v : 0.0;
+        LagT row[M];
+#pragma unroll
+        for (int l = 0; l < M; ++l)
+            row[l] = lag[off + min(l, nm - 1)];
+        __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+        for (int l = 0; l < M; ++l)
+            lam[l] = (l < nm) ? (l ? 2.0 : 1.0) * (double)row[l] : 0.0;
+    }
+    else
+    {
+#pragma unroll
+        for (int l = 0; l < M; ++l)
+        {
+            const LagT v = lag[off + min(l, nm - 1)];
+            lam[l] = (l < nm) ? (l ? 2.0 : 1.0) * (double)v : 0.0;
+        }
     }
     block_coefficients<M>(lam);
     float blo = 0.f, bhi = 1.f;
@@ -759,13 +778,17 @@ __global__ __launch_bounds__(256, 2) void reconstruct_adjoint_kernel(
             constexpr bool kProducts = K == 1 && M <= 40;
             using LamT = typename std::conditional<K == 1, double, float>::type;
             using GradT = typename std::conditional<kProducts, double, float>::type;
+            float row[M]; // unconditional loads before their use, as in the forward
+#pragma unroll
+            for (int l = 0; l < M; ++l)
+                row[l] = lag[off + min(j0 + l, nm - 1)];
+            __builtin_amdgcn_sched_barrier(0);
             LamT lam[M];
             GradT glam[M];
 #pragma unroll
             for (int l = 0; l < M; ++l)
             {
-                const float v = lag[off + min(j0 + l, nm - 1)]; // unconditional, as in the forward
-                lam[l] = (j0 + l < nm) ? (LamT)v * (LamT)((K == 1 && l > 0) ? 2 : 1) : (LamT)0;
+                lam[l] = (j0 + l < nm) ? (LamT)row[l] * (LamT)((K == 1 && l > 0) ? 2 : 1) : (LamT)0;
                 glam[l] = (GradT)0;
             }
             if constexpr (K == 1)
