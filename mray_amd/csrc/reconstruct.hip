@@ -14,9 +14,11 @@
 //         as the reference CPU path.
 //
 //  MIXED  multipliers in registers (template M >= m); the series
-//         lambda_0 + 2 sum_l lambda_l cos(l theta) by Clenshaw's recurrence
-//         in FP64 (2 VALU ops per term, cos theta from an FP64 sine of the
-//         half angle per sample): at 50 moments the multipliers reach
+//         lambda_0 + 2 sum_l lambda_l cos(l theta) in FP64, as products of
+//         Chebyshev polynomials of two orders (cheb_blocks.hpp, about 1.3 VALU
+//         ops per term; above 128 moments Clenshaw's recurrence over the
+//         lanes' chunks), cos theta from an FP64 sine of the half angle per
+//         sample: at 50 moments the multipliers reach
 //         |lambda| ~ 1e3 and an FP32 series loses ~1e-4 of density to
 //         cancellation, while FP64 FMAs cost the same issue slots as FP32
 //         ones on gfx950. The 256-entry transfer function is staged in LDS
@@ -477,7 +479,7 @@ __device__ __forceinline__ void chunk_starts(double x, double (&tn)[4], double (
 // multipliers split over K adjacent lanes (lane k holds lambda_64k ..
 // lambda_64k+63 in lam, zero past the pixel's count): each lane's Clenshaw
 // sum over its chunk from T_64k, T_64k-1 of the shared x = cos(theta) (taken
-// from the half angle as in series_clenshaw), the K partial sums added by an
+// from the half angle, cos_theta_of), the K partial sums added by an
 // xor butterfly, so every lane of the ray gets the same value bit for bit.
 // Also returns x and the lane's T_64k, T_64k-1 (for the reverse's forward
 // recurrence over its chunk).
@@ -662,21 +664,25 @@ __device__ __forceinline__ float fast_atan_deriv(float t)
 // entries from fs and its weight from frac(256 bs), so only bs carries a
 // derivative: d c / d bs = 256 (T[x1] - T[x0]). Then
 // d rho / d S = fast_atan'(S) / pi (hi - lo) and dS / d lambda_l = c_l cos(l theta)
-// (c_0 = 1, c_l = 2): FP64 sums of products (block_sums), rounded to float once.
+// (c_0 = 1, c_l = 2): up to 40 moments FP64 sums of products (block_sums),
+// rounded to float once; above, FP32 sums by the Chebyshev recurrence.
 // Transfer-function gradients are summed per workgroup in LDS and added to
 // grad_tf with one atomic per entry and workgroup. The LDS sums are 64-bit
 // fixed point (integer atomics: float atomics on LDS cost several times as
 // much here, above all when the rays of a wavefront add to the same entry);
 // the workgroup's scale 2^kfix comes from a bound on what each ray can add to
 // one entry, so that no partial sum reaches 2^61.
-
+// Registers: two wavefronts per SIMD up to 60 moments (60 itself with 13
+// spills); with 64 multipliers per lane the spills of a second one cost more
+// than it gives, above all in small images (64 x 48 rays, 128 moments: 233 us
+// by one, 359 by two; 512 x 512, 64 moments: 855 and 800).
 
 // K > 1: K adjacent lanes per ray (M = 64 multipliers each, as
 // reconstruct_mixed_split_kernel): every lane recomputes the ray's march with
 // the shared series value, accumulates the gradient of its own multipliers,
 // and only lane 0 adds to the table gradient.
 template <int M, int K = 1>
-__global__ __launch_bounds__(256, 2) void reconstruct_adjoint_kernel(
+__global__ __launch_bounds__(256, (K == 1 && M <= 60) ? 2 : 1) void reconstruct_adjoint_kernel(
     DevCamera cam, RecArgs a, const float *__restrict__ lag, const uint32_t *__restrict__ index,
     const uint32_t *__restrict__ bounds, const float4 *__restrict__ tf_g, const float4 *__restrict__ rgba_fwd,
     const float4 *__restrict__ grad_rgba, float *__restrict__ grad_lag, float *__restrict__ grad_tf)
@@ -782,7 +788,8 @@ __global__ __launch_bounds__(256, 2) void reconstruct_adjoint_kernel(
 #pragma unroll
             for (int l = 0; l < M; ++l)
                 row[l] = lag[off + min(j0 + l, nm - 1)];
-            __builtin_amdgcn_sched_barrier(0);
+            if constexpr (K == 1)
+                __builtin_amdgcn_sched_barrier(0);
             LamT lam[M];
             GradT glam[M];
 #pragma unroll
@@ -981,6 +988,7 @@ int launch_reconstruct_adjoint(const mray_camera &cam, const float *dmin, const 
     MRAY_ADJ_CASE(40)
     MRAY_ADJ_CASE(48)
     MRAY_ADJ_CASE(56)
+    MRAY_ADJ_CASE(60)
     MRAY_ADJ_CASE(64)
 #undef MRAY_ADJ_CASE
     // 65..256: two or four lanes per ray, 64 multipliers each
