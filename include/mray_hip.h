@@ -88,8 +88,13 @@ const void *mray_hip_volume_data(mray_volume vol);
  *                were normalised with (before the 16-bit packing of
  *                d_bounds), for mray_hip_generate_backward; NULL to skip
  * form: MRAY_FORM_PLAIN or MRAY_FORM_MIXED (m up to 255 in both; MIXED splits
- * more than 64 moments into chunks of at most 56, each marched by its own
- * workgroups). Compaction and prediction coding
+ * more than 60 moments into chunks of at most 50, each marched by its own
+ * workgroups). MIXED sums a grid volume's moments with or without d_ray_range
+ * by two forms of the same FP64 sums: with it every ray node by node (the
+ * forward of a gradient, which the reverse of the preparation would otherwise
+ * see a change of rounding in), without it on the grid of the ray's phases
+ * where its samples resolve the moments, which is faster. The moments differ
+ * by their float rounding. Compaction and prediction coding
  * are separate calls (mray_hip_compute_num_moments, mray_hip_moment_index,
  * mray_hip_compact, mray_hip_prediction_encode). */
 int mray_hip_generate(mray_volume vol, const mray_camera *cam, const mray_gen_params *p, int form, int W, int H,
@@ -407,7 +412,9 @@ int mray_hip_entropy_decode(const uint8_t *h_in, size_t n_in, const uint32_t *d_
  * values of particles closer than h. Particles are ordered by cell with a
  * stable sort, so the result is deterministic. Synchronises the stream once
  * (the cell grid is sized from the particles' bounding box); uses
- * stream-ordered scratch of about 28 bytes per particle + 8 per cell. */
+ * stream-ordered scratch of about 56 bytes per particle + 8 per cell: 16 for
+ * the sorted records, 40 more while they are sorted (32 and the radix sort's
+ * own, in one allocation). */
 int mray_hip_particles_to_grid(const float *d_x, const float *d_y, const float *d_z, const float *d_v, uint32_t n,
                                float h, const float dom_min[3], const float dom_max[3], int nx, int ny, int nz,
                                float *d_grid, mray_stream stream);

@@ -76,11 +76,13 @@ class GenerateFunction(torch.autograd.Function):
     @staticmethod
     def forward(ctx, voxels, dmin, dmax, cam, gp, W, H, m):
         vol = hip.Volume(voxels.detach().contiguous(), dmin, dmax)
-        # the per-ray normalisation is kept for the reverse pass
-        rr = torch.empty((H * W, 2), dtype=torch.float32, device=voxels.device) if gp.transform_to_bounds else None
+        # the per-ray normalisation is kept for the reverse pass; asked for also
+        # where nothing is normalised (transform_to_bounds = 0): a call that
+        # records it sums every ray's moments node by node
+        rr = torch.empty((H * W, 2), dtype=torch.float32, device=voxels.device)
         mo, bounds, _ = hip.generate(vol, cam, gp, W, H, m, form="mixed", ray_range=rr)
         ctx.vol = vol
-        ctx.ray_range = rr
+        ctx.ray_range = rr if gp.transform_to_bounds else None
         ctx.args = (cam, gp, W, H, m)
         ctx.mark_non_differentiable(bounds) if bounds is not None else None
         return mo, bounds

@@ -195,7 +195,9 @@ class ParticleVolume(Volume):
 def generate(vol: Volume, cam: dict, gp: GenParams, W: int, H: int, m: int, form="mixed", moments=None,
              bounds=None, samples=None, want_samples=False, ray_range=None, stream=None):
     """Dense moments (H, W, m), packed bounds (H*W,) uint32 (or None), samples per ray (or None).
-    ray_range: optional (H*W, 2) float32 tensor that receives each ray's normalisation (lo, hi)."""
+    ray_range: optional (H*W, 2) float32 tensor that receives each ray's normalisation (lo, hi);
+    with it a mixed call sums every ray's moments node by node, without it most rays on the
+    grid of their phases (mray_hip_generate: last bits and speed differ)."""
     dev = vol.voxels.device if vol.voxels is not None else vol._parts[0].device
     if moments is None:
         moments = torch.empty((H, W, m), dtype=torch.float32, device=dev)

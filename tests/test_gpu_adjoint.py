@@ -547,3 +547,26 @@ def test_render_autograd_chain(hip):
         l2 = float(((ag.render(x2, dmin, dmax, cam, gp, W, H, m, table, rp) - target) ** 2).sum())
     print(f"[render autograd] loss {float(loss):.6e} -> {l2:.6e} after a step of 1e-3 against the gradient")
     assert l2 < float(loss)
+
+
+@pytest.mark.parametrize("bounded", [0, 1])
+def test_gradient_forward_is_summed_node_by_node(bounded):
+    """The forward of a gradient takes the march that records the rays'
+    normalisation, also where no moment is normalised: its moments are the bits
+    of a call with ray_range."""
+    import torch
+
+    from mray_amd import autograd as ag, hip, synth
+    from mray_amd.types import GenParams
+
+    n, W, H, m = 48, 70, 50, 24
+    vox = torch.from_numpy(synth.mixing_layer(n, width=0.05)).cuda()
+    cam = synth.perspective_camera(aspect=W / H)
+    gp = GenParams(step_size=0.25 / n, transform_to_bounds=bounded, transform_bound_eps=0.01, compact_image=0,
+                   prediction_coding=0, bias=1e-4)
+    rr = torch.empty((H * W, 2), dtype=torch.float32, device="cuda")
+    ref, _, _ = hip.generate(hip.Volume(vox, (0,) * 3, (1,) * 3), cam, gp, W, H, m, ray_range=rr)
+    mo, _ = ag.GenerateFunction.apply(vox.requires_grad_(True), (0,) * 3, (1,) * 3, cam, gp, W, H, m)
+    assert torch.equal(mo.detach(), ref)
+    mo.sum().backward()
+    assert torch.isfinite(vox.grad).all() and float(vox.grad.abs().max()) > 0
