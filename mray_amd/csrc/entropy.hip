@@ -37,6 +37,7 @@
 #include <vector>
 
 #include "device_common.hpp"
+#include "digit_ring.hpp"
 #include "fastac_lanes.hpp"
 #include "launch.hpp"
 
@@ -267,75 +268,58 @@ __device__ __forceinline__ uint64_t first_bits(uint64_t mask, uint32_t k)
     return out;
 }
 
+// DigitRing's operations on a wavefront
+struct DeviceWave
+{
+    using u32 = uint32_t;
+    static __device__ __forceinline__ bool first() { return threadIdx.x == 0; }
+    static __device__ __forceinline__ void add(uint32_t *p, uint32_t v) { atomicAdd(p, v); }
+    static __device__ __forceinline__ void sync() { __syncthreads(); }
+    static __device__ __forceinline__ void fence() { __threadfence(); }
+    static __device__ __forceinline__ u32 load(const uint32_t *ring, uint32_t at, uint32_t n)
+    {
+        return (threadIdx.x < n) ? ring[(at + threadIdx.x) & 127u] : 0u;
+    }
+    static __device__ __forceinline__ bool any_above(u32 v, uint32_t top) { return __ballot(v > top) != 0ull; }
+    static __device__ __forceinline__ u32 shift_right(u32 v, int k) { return v >> k; }
+    static __device__ __forceinline__ u32 low_bits(u32 v, uint32_t mask) { return v & mask; }
+    static __device__ __forceinline__ u32 plus(u32 a, u32 b) { return a + b; }
+    static __device__ __forceinline__ uint32_t lane0(u32 v)
+    {
+        return (uint32_t)__builtin_amdgcn_readfirstlane((int)v);
+    }
+    // the next lane's value, 0 in the last
+    static __device__ __forceinline__ u32 from_next(u32 v)
+    {
+        const u32 up = __shfl_down(v, 1);
+        return threadIdx.x < 63u ? up : 0u;
+    }
+    // the first n lanes' digits as bytes from out + at, up to cap
+    static __device__ __forceinline__ void store(uint8_t *out, size_t cap, size_t at, u32 v, uint32_t n)
+    {
+        const uint32_t lane = threadIdx.x;
+        const size_t p = at + 2 * (size_t)lane;
+        if (lane < n)
+        {
+            if (p < cap)
+                out[p] = (uint8_t)(v >> 8);
+            if (p + 1 < cap)
+                out[p + 1] = (uint8_t)v;
+        }
+    }
+};
+
 // The encoder's state (Arithmetic_Codec in mode 1): the interval, and the code
-// as 16-bit digits (a renormalisation shifts out two bytes). The newest digits
-// are in an LDS ring of 128; a carry adds 1 to the newest one without looking
-// at it, and the digits are brought into [0, 2^16) when 64 of them leave the
-// ring together (flush). The newest digit always stays, so that a carry finds
-// its digit in the ring.
 struct Encoder
 {
     double base, length;
-    uint8_t *out;
-    size_t cap;
-    uint32_t *ring;        // 128 digits in LDS
-    uint32_t nd, flushed;  // digits so far, and of them in out
-
-    __device__ __forceinline__ void put(uint32_t a)
-    {
-        if (threadIdx.x == 0)
-            ring[nd & 127u] = a;
-        ++nd;
-        if (nd - flushed >= 96u)
-            flush(64u);
-    }
+    DigitRing<DeviceWave> digits;
 
     // propagate_carry (src/entropy_coding/arithmetic_codec.cpp:76-84)
     __device__ __forceinline__ void carry()
     {
         base -= 1.0;
-        if (threadIdx.x == 0 && nd > 0)
-            atomicAdd(&ring[(nd - 1u) & 127u], 1u);
-    }
-
-    // the next n <= 64 digits of the ring to out
-    __device__ __forceinline__ void flush(uint32_t n)
-    {
-        __syncthreads();
-        const uint32_t lane = threadIdx.x;
-        uint32_t v = (lane < n) ? ring[(flushed + lane) & 127u] : 0u;
-        uint32_t carried = 0;
-        while (__ballot(v > 0xFFFFu))
-        {
-            const uint32_t c = v >> 16;
-            carried += (uint32_t)__builtin_amdgcn_readfirstlane((int)c);
-            const uint32_t up = __shfl_down(c, 1);
-            v = (v & 0xFFFFu) + (lane < 63u ? up : 0u);
-        }
-        const size_t at = 2 * (size_t)(flushed + lane);
-        if (carried)
-        {
-            // into the bytes already out
-            __threadfence();
-            if (lane == 0)
-            {
-                size_t p = 2 * (size_t)flushed - 1;
-                while (p < cap && out[p] == 0xFFu)
-                    out[p--] = 0;
-                if (p < cap)
-                    out[p] = (uint8_t)(out[p] + 1);
-            }
-            __threadfence();
-        }
-        if (lane < n)
-        {
-            if (at < cap)
-                out[at] = (uint8_t)(v >> 8);
-            if (at + 1 < cap)
-                out[at + 1] = (uint8_t)v;
-        }
-        flushed += n;
-        __syncthreads();
+        digits.carry();
     }
 
     // encode(data, Adaptive_Data_Model) with the symbol's d(s) and d(s + 1)
@@ -356,7 +340,7 @@ struct Encoder
             {
                 base *= kOut;
                 const uint32_t a = (uint32_t)base;
-                put(a);
+                digits.put(a);
                 base -= (double)a;
                 length *= kOut;
             }
@@ -385,15 +369,14 @@ struct Encoder
         }
         if (base >= 1.0)
             carry();
-        while (flushed < nd)
-            flush(min(64u, nd - flushed));
-        size_t pos = 2 * (size_t)nd;
+        digits.flush_all();
+        size_t pos = 2 * (size_t)digits.nd;
         do
         {
             base *= 256.0;
             const uint32_t c = (uint32_t)base;
-            if (threadIdx.x == 0 && pos < cap)
-                out[pos] = (uint8_t)c;
+            if (threadIdx.x == 0 && pos < digits.cap)
+                digits.out[pos] = (uint8_t)c;
             ++pos;
             base -= (double)c;
         } while (--last);
@@ -440,7 +423,7 @@ __global__ __launch_bounds__(64) void entropy_encode_kernel(const float *__restr
     Model M;
     M.reset(lds_model, 1u << bits);
     __shared__ uint32_t ring[128];
-    Encoder E{0.0, 1.0, streams + stream_off[l - 1], (size_t)(stream_off[l] - stream_off[l - 1]), ring, 0u, 0u};
+    Encoder E{0.0, 1.0, {streams + stream_off[l - 1], (size_t)(stream_off[l] - stream_off[l - 1]), ring, 0u, 0u}};
     for (uint32_t p0 = 0; p0 < npix; p0 += 64)
     {
         const uint32_t p = p0 + lane;
@@ -480,7 +463,7 @@ __global__ __launch_bounds__(64) void entropy_encode_kernel(const float *__restr
     }
     const size_t size = E.finish();
     if (lane == 0)
-        sizes[l] = size > E.cap ? ~0ull : (uint64_t)size;
+        sizes[l] = size > E.digits.cap ? ~0ull : (uint64_t)size;
 }
 
 // The decoder's state (Arithmetic_Codec in mode 2); bytes past the code's

@@ -674,8 +674,8 @@ __device__ __forceinline__ float fast_atan_deriv(float t)
 // one entry, so that no partial sum reaches 2^61.
 // Registers: two wavefronts per SIMD up to 60 moments (60 itself with 13
 // spills); with 64 multipliers per lane the spills of a second one cost more
-// than it gives, above all in small images (64 x 48 rays, 128 moments: 233 us
-// by one, 359 by two; 512 x 512, 64 moments: 855 and 800).
+// than it gives, above all in small images (64 x 48 rays, 128 moments: 239 us
+// by one, 360 by two; 512 x 512, 64 moments: 855 and 802).
 
 // K > 1: K adjacent lanes per ray (M = 64 multipliers each, as
 // reconstruct_mixed_split_kernel): every lane recomputes the ray's march with
