@@ -13,7 +13,7 @@
 //         the Toeplitz solve in FP64, where conditioning at 50+ moments needs
 //         it; the autocorrelation and correlation stay FP64 too since FP64
 //         FMA is full rate on gfx950. Four lanes work on a pixel (8 or 16
-//         above 104 moments), its arrays in registers (mese_lattice.hpp).
+//         above 100 moments or in small images), its arrays in registers (mese_lattice.hpp).
 //         The reflection coefficients come from Schur's recursion on the
 //         moments instead of Levinson's inner products, together with the
 //         solution polynomial in one lattice (see the kernel).
@@ -78,7 +78,7 @@ __global__ __launch_bounds__(64) void prepare_plain_kernel(const float *__restri
 // this one 1.92 (VALU issue in 96 % of the cycles); a compact 1000 x 777 image
 // of 8 to 96 moments 6.8 and 2.85 ms. G = 4 makes the
 // share of the per-step overhead small (16 pixels per wavefront) while the two
-// arrays fit the registers of two wavefronts per SIMD (C <= 26).
+// arrays fit the registers of two wavefronts per SIMD (C <= 25).
 // OutT: float multipliers, or FP64 ones for mray_hip_prepare_f64
 template <int G, int C, typename OutT>
 __global__ __launch_bounds__(64, 2) void prepare_mixed_kernel(const float *__restrict__ mom,

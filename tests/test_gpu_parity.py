@@ -266,13 +266,13 @@ def test_prepare_parity(hip, O, name, form):
 
 
 @pytest.mark.parametrize("m", [64, 72, 80, 88, 100, 128, 160, 200, 248, 255])
-def test_prepare_mixed_large_m(hip, O, m):
-    """MIXED preparation beyond the parity cases' 50 moments, up to 255 (16
-    element slots per lane up to 128, then 20-32; at 10, 11, 13, 20 and 32
-    slots, 80, 88, 100, 160 and 255 moments here, the per-pixel LDS arrays
-    have no bank padding): densities against the FP64
-    oracle at 41 phases with the float-storage bound of test_prepare_parity.
-    Moments from the oracle's generate."""
+@pytest.mark.parametrize("copies", [1, 50, 80])
+def test_prepare_mixed_large_m(hip, O, m, copies):
+    """MIXED preparation beyond the parity cases' 50 moments, up to 255, in images
+    of up to 4096, up to 8192 and more pixels (16, 8 and 4 lanes per pixel where
+    those hold the moments): densities against the FP64 oracle at 41 phases with
+    the float-storage bound of test_prepare_parity. Moments from the oracle's
+    generate, the same image `copies` times over."""
     import torch
 
     vol = synth.marschner_lobb(32)
@@ -284,7 +284,10 @@ def test_prepare_mixed_large_m(hip, O, m):
     print(f"[prepare large m] m={m} W={W} H={H}", flush=True)
     mo_ref, _, ns_ref = O.generate(vol, dmin, dmax, cam, W, H, m, gp)
     bias = 5e-5
-    lag = to_np(hip.prepare(torch.from_numpy(mo_ref).cuda(), W, H, m, bias, form="mixed")).reshape(-1, m)
+    lag = to_np(hip.prepare(torch.from_numpy(mo_ref).cuda().repeat(copies, 1, 1), W, H * copies, m, bias,
+                            form="mixed")).reshape(copies, -1, m)
+    assert np.array_equal(lag, np.broadcast_to(lag[0], lag.shape))
+    lag = lag[-1]
     phases = np.linspace(-np.pi, 0.0, 41)
     worst = -1.0
     for p in np.nonzero(ns_ref > 0)[0][::4]:

@@ -4,10 +4,11 @@
 Both solve the same Toeplitz system in FP64, so at MESE bias 1e-3 and these
 densities (|u|^2 up to ~0.99) multipliers agree to a small multiple of the
 conditioning times 2^-53; the bound is 1e-9 of a pixel's largest multiplier
-(f32 multipliers: half an ulp more). Counts at the edges of the lanes' blocks
-(4, 8 and 16 lanes per pixel, by image size and by moments), compact images of
-ragged counts with empty pixels, and moments outside the moment space, where
-the |u|^2 >= 1 guard fires and every later coefficient is 0."""
+(f32 multipliers: half an ulp more). Every kernel of the dispatch (4, 8 and 16
+lanes per pixel, by image size and by moments) at the edges of its width, dense
+and in compact images of ragged counts with empty pixels, and moments outside
+the moment space, where the |u|^2 >= 1 guard fires and every later coefficient
+is 0."""
 import numpy as np
 import pytest
 import torch
@@ -43,14 +44,47 @@ def check(O, mo, lag, nm, bias, tol):
         assert np.abs(lag[i][:nm[i]] - ref).max() <= tol * np.abs(ref).max(), (i, nm[i])
 
 
-# images of up to 4096, up to 8192 and more pixels take 16, 8 and 4 lanes
-@pytest.mark.parametrize("W,H", [(9, 7), (64, 64), (65, 64), (128, 64), (129, 64)])
-@pytest.mark.parametrize("m", [1, 2, 7, 8, 9, 31, 33, 50, 100, 101, 129, 193, 255])
+# The widths of the dispatch, lanes x elements per lane: images of up to 4096,
+# up to 8192 and more pixels take 16, 8 and 4 lanes where that many hold the
+# moments, else more.
+ELEMENTS = {16: (2, 3, 4, 5, 6, 7, 8, 10, 13, 16), 8: (2, 3, 4, 5, 6, 7, 8, 10, 13),
+            4: (2, 3, 4, 5, 6, 7, 8, 9, 10, 11, 12, 13, 14, 15, 16, 18, 20, 22, 24, 25)}
+BEYOND_FOUR = tuple(8 * c for c in (16, 20, 24)) + (16 * 13, 16 * 16)
+SIZES = {16: ((9, 7), (64, 64)), 8: ((65, 64), (128, 64)), 4: ((129, 64),)}
+
+
+def widths(lanes):
+    own = tuple(lanes * c for c in ELEMENTS[lanes])
+    return own + tuple(w for w in BEYOND_FOUR if w > own[-1])
+
+
+def edges(lanes):
+    """Each width full, short of one moment, and one past the width before."""
+    w = widths(lanes)
+    return sorted({m for lo, hi in zip((0,) + w, w) for m in (lo + 1, hi - 1, hi) if m <= 255})
+
+
+def cases():
+    for lanes, sizes in SIZES.items():
+        for m in edges(lanes):
+            yield sizes[-1] + (m,)
+        for size in sizes[:-1]:
+            for m in (1, 2, 7, 8, 33, 50, 100, 101, 129, 193, 255):
+                yield size + (m,)
+
+
+def ragged(rng, n, m):
+    nm = rng.integers(0, m + 1, n)
+    nm[:40] = np.arange(40) % (m + 1)
+    nm[-3:] = (0, 1, m)
+    return nm
+
+
+@pytest.mark.parametrize("W,H,m", list(cases()))
 def test_dense(O, W, H, m):
-    if W * H > 100 and m not in (8, 33, 50, 100, 101):
-        pytest.skip("edges of the lane blocks are covered at the smallest size")
     rng = np.random.default_rng(W * 1000 + m)
-    mo = densities(rng, W * H, m)
+    few = densities(rng, min(W * H, 64), m)
+    mo = few[np.arange(W * H) % len(few)]
     lag = hip.prepare(torch.from_numpy(mo).cuda(), W, H, m, 1e-3, form="mixed64").cpu().numpy().reshape(-1, m)
     pick = np.unique(np.concatenate([np.arange(3), rng.integers(0, W * H, 12), np.arange(W * H - 3, W * H)]))
     check(O, mo[pick], lag[pick], np.full(len(pick), m), 1e-3, 1e-9)
@@ -58,14 +92,30 @@ def test_dense(O, W, H, m):
     assert np.array_equal(f32, lag.astype(np.float32))
 
 
+@pytest.mark.parametrize("lanes", [16, 8, 4])
+def test_compact_matches_dense(O, lanes):
+    """Ragged counts through every kernel of the dispatch: a pixel of n moments
+    gets what an image of n moments gives it, up to the padding's zeros."""
+    W, H = SIZES[lanes][-1]
+    rng = np.random.default_rng(lanes)
+    for m in (w for w in widths(lanes) if w <= 255):
+        mo = densities(rng, 64, m)[np.arange(W * H) % 64]
+        nm = ragged(rng, W * H, m)
+        index = np.concatenate([[0], np.cumsum(nm)]).astype(np.int32)
+        data = mo[np.arange(m)[None] < nm[:, None]]
+        lag = hip.prepare(torch.from_numpy(data).cuda(), W, H, m, 1e-3, form="mixed64",
+                          index=torch.from_numpy(index).cuda()).cpu().numpy()
+        pick = np.unique(np.concatenate([np.arange(1, 6), rng.integers(0, W * H, 6), np.arange(W * H - 2, W * H)]))
+        pick = pick[nm[pick] > 0]
+        check(O, mo[pick], [lag[index[i]:index[i + 1]] for i in pick], nm[pick], 1e-3, 1e-9)
+
+
 @pytest.mark.parametrize("W,H", [(12, 11), (70, 70), (130, 64)])
 def test_compact_ragged(O, W, H):
     m = 60
     rng = np.random.default_rng(W)
     mo = densities(rng, W * H, m)
-    nm = rng.integers(0, m + 1, W * H)
-    nm[:40] = np.arange(40) % (m + 1)
-    nm[-3:] = (0, 1, m)
+    nm = ragged(rng, W * H, m)
     index = np.concatenate([[0], np.cumsum(nm)]).astype(np.int32)
     data = np.concatenate([mo[i][:nm[i]] for i in range(W * H)])
     lag = hip.prepare(torch.from_numpy(data).cuda(), W, H, m, 1e-3, form="mixed64",
