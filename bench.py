@@ -368,6 +368,8 @@ def main():
         "roofline": {"bound": "valu", "kernel": dom, "achieved": round(achieved / 1e12, 3),
                      "peak": PEAK_FP32_VALU / 1e12, "unit": "TFLOP/s",
                      "frac": round(achieved / PEAK_FP32_VALU, 4),
+                     "flops": "credited: 8 (m - 1) + 30 or 48 a sample and 20 m^2 a pixel, more than the mixed "
+                              "kernels execute; frac is no share of what the chip's VALUs issued",
                      "traffic": measured_traffic(dom, n, W, m)},
         "roofline_frame": {"achieved_TFLOPs": round(total_flop / (ms_step * 1e-3) / 1e12, 3),
                            "frac": round(total_flop / (ms_step * 1e-3) / PEAK_FP32_VALU, 4)},
