@@ -404,16 +404,18 @@ template <int CTRL> __device__ __forceinline__ double dpp_quad(double v)
 // of them spilled cost less than the third wavefront is worth (128^3 f32, 509 x
 // 387 rays, 30 moments: 350 us by two, 320 by three; in a domain of 0.9^3 396
 // and 422). Node by node 30 moments come to 170 to 174 (512 x 512 rays, 487 and
-// 460 us); particle sets are better off without (1229 and 1363 us).
-template <typename T, int M, bool POW2, bool GRID, int S> constexpr int mixed_wavefronts()
+// 460 us). Particle sets and volumes beyond 32-bit offsets, whose samples wait
+// on memory, are better off without (node by node 1229 and 1363 us, 1100^3
+// voxels 836 and 948; 28 moments on the grid 867 and 1008).
+template <typename T, int M, bool OFF32, bool POW2, bool GRID, int S> constexpr int mixed_wavefronts()
 {
     if (!GRID)
-        return (M == 30 && !std::is_same<T, SphParticle>::value) ? 3 : 1;
-    return (S == 1 && M <= (POW2 ? 30 : 28)) ? 3 : 2;
+        return (M == 30 && OFF32 && !std::is_same<T, SphParticle>::value) ? 3 : 1;
+    return (S == 1 && M <= (!OFF32 ? 24 : POW2 ? 30 : 28)) ? 3 : 2;
 }
 
 template <typename T, int M, bool OFF32, bool POW2, bool CHUNK, bool GRID, int J0C, int S = 1>
-__global__ __launch_bounds__(256, (mixed_wavefronts<T, M, POW2, GRID, S>())) void generate_mixed_kernel(VolumeView<T> vol, DevCamera cam, GenArgs a,
+__global__ __launch_bounds__(256, (mixed_wavefronts<T, M, OFF32, POW2, GRID, S>())) void generate_mixed_kernel(VolumeView<T> vol, DevCamera cam, GenArgs a,
                                                              float *__restrict__ out, uint32_t *__restrict__ bounds,
                                                              int32_t *__restrict__ samples,
                                                              float2 *__restrict__ ray_range)
