@@ -307,9 +307,11 @@ __global__ __launch_bounds__(256) void reconstruct_mixed_kernel(DevCamera cam, R
     // the coefficients' sums, which begin with the last, the loads spread out
     // (1024 x 1024 rays, 30 moments: 141 us of the call, 48 now; FP64
     // multipliers 232 and 50). Above 96 the registers don't hold a row in
-    // flight beside the multipliers (104, 512 x 512 rays: 321 us, 353 with it).
+    // flight beside the multipliers (104, 512 x 512 rays: 321 us, 353 with it),
+    // and few rays leave the loads no cache to miss (S = 4, 60 x 50 rays of 700
+    // steps, 22 moments: 100 us, 106 with it).
     double lam[M];
-    if constexpr (kTwoSteps<M>)
+    if constexpr (kTwoSteps<M> && S == 1)
     {
         LagT row[M];
 #pragma unroll
