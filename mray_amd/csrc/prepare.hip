@@ -75,7 +75,7 @@ __global__ __launch_bounds__(64) void prepare_plain_kernel(const float *__restri
 // A step costs 8 C FMAs and about 35 operations for k, the seam, two
 // broadcasts and the shift, none of them LDS: at 50 moments (1024 x 1024
 // pixels, FP64 multipliers) the LDS-bound Levinson kernel before took 4.37 ms,
-// this one 1.92 (VALU issue in 96 % of the cycles); a compact 1000 x 777 image
+// this one 1.92 (VALU issue in 85 to 89 % of the cycles); a compact 1000 x 777 image
 // of 8 to 96 moments 6.8 and 2.85 ms. G = 4 makes the
 // share of the per-step overhead small (16 pixels per wavefront) while the two
 // arrays fit the registers of two wavefronts per SIMD (C <= 25).
