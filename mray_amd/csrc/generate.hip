@@ -16,8 +16,8 @@
 //         The reference's segments are [p_k - dphi, p_k] with p_k recomputed
 //         from t, so neighbours overlap by a few ulp (delta), and its lines
 //         use the slope (f_k - f_{k-1}) / dphi, so they miss f_k by a few ulp
-//         (eps); both enter to first order, exactly enough to reproduce the
-//         reference's arithmetic-free result to ~1e-13:
+//         (eps); both enter to first order, their squares are ~1e-13 (more
+//         where t is thousands of steps, see GridStep):
 //             + sum_k [ -delta_k f_k cos(j p_k) + h_k sin(j p_k) / j ].
 //         Two marches sum these terms. Where the samples resolve the largest
 //         order (almost every ray), the ulp-sized terms become weights of
@@ -345,13 +345,29 @@ template <int CTRL> __device__ __forceinline__ double dpp_quad(double v)
     return __builtin_bit_cast(double, w);
 }
 
+// wavefronts per SIMD a kernel's registers are held to. Up to 30 moments (28 in
+// general domains) a GRID kernel comes to 168 to 184 without a bound, and 3 to 14
+// of them spilled cost less than the third wavefront is worth (128^3 f32, 509 x
+// 387 rays, 30 moments: 350 us by two, 320 by three; in a domain of 0.9^3 396
+// and 422). Node by node 30 moments come to 170 to 174 (512 x 512 rays, 487 and
+// 460 us). Particle sets and volumes beyond 32-bit offsets, whose samples wait
+// on memory, are better off without (node by node 1229 and 1363 us, 1100^3
+// voxels 836 and 948; 28 moments on the grid 867 and 1008).
+template <typename T, int M, bool OFF32, bool POW2, bool GRID, int S> constexpr int mixed_wavefronts()
+{
+    if (!GRID)
+        return (M == 30 && OFF32 && !std::is_same<T, SphParticle>::value) ? 3 : 1;
+    return (S == 1 && M <= (!OFF32 ? 24 : POW2 ? 30 : 28)) ? 3 : 2;
+}
+
 // The integral per node. A segment [u, p] of the reference with slope g
 // contributes, with c(phi) = cos(j phi) and rho the line's values at its ends,
 //     (1/j^2) [ g c(p) - rho_p c'(p) - g c(u) + rho_u c'(u) ].
 // Node k gathers the end of segment k (at p_k) and the start of segment k + 1
 // (at u_k+1 = p_k + delta, the reference's p_k+1 - dphi in float). Expanded
 // around the uniform grid q_k = (t_k - t_near) pi / range - pi (p_k = q_k +
-// eps; eps, delta are a few float ulps of the phase, their squares ~1e-13):
+// eps; eps, delta are a few float ulps of the phase, their squares ~1e-13, and
+// next to 8192 steps from t = 0 delta is up to 2^-12 of dphi: GridStep):
 //     d c + cp c' + cpp c''   at q_k,
 //     d   = g_k - g_k+1
 //     cp  = d eps - g_k+1 delta - g_k (width_k - dphi)
@@ -398,22 +414,8 @@ template <int CTRL> __device__ __forceinline__ double dpp_quad(double v)
 // Measured (1024^3 f32, 1024 x 1024 rays, 50 moments): 11.6 ms node by node,
 // 7.1 ms gridded (8.1 before the corners came in pairs); 2048 x 2048 x 1920
 // u8, 2048 x 2048 rays, 100 moments: 132 and 76 ms (the bytes' divisions and
-// the corner addresses are a third of that gain). Bound by VALU issue, then by load latency at two wavefronts per SIMD.
-// wavefronts per SIMD a kernel's registers are held to. Up to 30 moments (28 in
-// general domains) a GRID kernel comes to 168 to 184 without a bound, and 3 to 14
-// of them spilled cost less than the third wavefront is worth (128^3 f32, 509 x
-// 387 rays, 30 moments: 350 us by two, 320 by three; in a domain of 0.9^3 396
-// and 422). Node by node 30 moments come to 170 to 174 (512 x 512 rays, 487 and
-// 460 us). Particle sets and volumes beyond 32-bit offsets, whose samples wait
-// on memory, are better off without (node by node 1229 and 1363 us, 1100^3
-// voxels 836 and 948; 28 moments on the grid 867 and 1008).
-template <typename T, int M, bool OFF32, bool POW2, bool GRID, int S> constexpr int mixed_wavefronts()
-{
-    if (!GRID)
-        return (M == 30 && OFF32 && !std::is_same<T, SphParticle>::value) ? 3 : 1;
-    return (S == 1 && M <= (!OFF32 ? 24 : POW2 ? 30 : 28)) ? 3 : 2;
-}
-
+// the corner addresses are a third of that gain). Bound by VALU issue, then by
+// load latency at two wavefronts per SIMD.
 template <typename T, int M, bool OFF32, bool POW2, bool CHUNK, bool GRID, int J0C, int S = 1>
 __global__ __launch_bounds__(256, (mixed_wavefronts<T, M, OFF32, POW2, GRID, S>())) void generate_mixed_kernel(VolumeView<T> vol, DevCamera cam, GenArgs a,
                                                              float *__restrict__ out, uint32_t *__restrict__ bounds,
